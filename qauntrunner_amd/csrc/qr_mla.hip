@@ -6,10 +6,12 @@
 //
 // mla_tile_kernel (bf16/f16 latents, kv_lora 512, rope 0 or 64): MFMA tiles, see
 //   below; splits merged by mla_combine_wide_kernel.
+// mla_f32_kernel (fp32 latents, kv_lora 256 or 512, rope 0, 32 or 64): fp32 MFMA tiles,
+//   see below; splits merged by mla_combine_f32_kernel.
 // mla_split_generic_kernel: one workgroup per (split of 256 positions, head).
 //   Scores of the split are staged in LDS; the split's partial (max, sum,
 //   unnormalised u) is merged across splits by mla_combine_kernel.  This path
-//   serves every other shape and the fp32 cache.
+//   serves every other shape.
 #include "qr_mla.hpp"
 #include "qr_mfma.hpp"
 
@@ -763,8 +765,321 @@ __global__ void __launch_bounds__(256) mla_combine_wide_kernel(const MlaMK p) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// fp32 MFMA path for fp32 latents (kv_lora 256 or 512, rope 0, 32 or 64).
+//
+// Bound by the fp32 MFMA rate (v_mfma_f32_16x16x4_f32, 256 flop per clk and CU, fp32 products
+// and sums as the generic kernel's FMAs): 128 heads over 4096 positions are 1.14 GFLOP, 7.4 us
+// at the 153 TFLOP/s of a large fp32 product.  The generic kernel read every row once per
+// head, one row per thread: 1092 us per call at that shape, this one with its merge 29.0
+// (25.9 + 4.0; two tiles per wave there, so the first loads of q~ and rows are half of it).
+// Error against 64-bit arithmetic there: 4.6e-7 (generic 1.4e-6).
+//
+// Workgroup = 16 heads over one split; its four waves take 16-position tiles 4i + w and work
+// alone: scores, online softmax and the latent sum of a tile stay in one wave, which the MFMA
+// layouts allow without any exchange of P.  Sixteen heads per workgroup (not 64, one tile for
+// four waves) keeps the splits few -- 32 at 128 heads -- and with them the fp32 partials that
+// the merge writes and reads (8.4 MB against 33.5); the rows are then read by every head
+// group, from the L2 of the XCD that the groups of one split share.
+//   QK  S^T[pos][head]: lane (q4, l16) holds dims 16j + 4q4 .. +3 of row l16 (A) and of head
+//       l16 (B), so k-slot q4 of MFMA e is dim 16j + 4q4 + e: both operands are 16-byte reads.
+//       A comes from the registers that the tile was loaded into, B from LDS (q~ scaled by
+//       scale log2 e, its last dims in registers where LDS is full).
+//   PV  U^T[dim][head]: lane quarter q4 holds the scores of positions 4q4 + r; step r takes
+//       those four positions as its k-slots, so P enters from the lane's own registers.  A is
+//       row 4q4 + r, dims 64g + 4 l16 + e: one 16-byte LDS read feeds the four MFMAs e.
+// A tile's rows go registers -> LDS (the wave's own 16 rows) once QK has used them, and the
+// next tile's loads fly during PV.  16-byte chunk c of an LDS row r sits at c ^ (r & 15).
+constexpr int kFHeads = 16;    // heads per workgroup
+constexpr int kFWaves = 4;
+constexpr int kFTile = 16;     // positions per wave and tile
+constexpr int kFStep = kFWaves * kFTile;
+constexpr int kFLds = 160 * 1024 - 1024;
+
+template <int KL, int KR>
+struct MlaF32Geom {
+    static constexpr int W = KL + KR;
+    static constexpr int NJ = W / 16;                    // QK steps of 16 dims
+    static constexpr int NV = KL / 16;                   // of them staged for PV
+    static constexpr int NG = KL / 64;                   // PV groups of 64 dims
+    static constexpr int VB = kFTile * KL * 4;           // bytes of a wave's staged rows
+    static constexpr int QFIT = (kFLds - kFWaves * VB) / (kFHeads * 256) * 64;  // dims of q~ that fit in LDS
+    static constexpr int QL = (QFIT < W ? QFIT : W) / 64 * 64;  // whole rounds of staging; the rest in registers
+    static constexpr int NJQ = QL / 16;                  // QK steps whose q~ is in LDS
+    static constexpr int QP = QL * 4;                    // bytes of a q~ row in LDS
+};
+
+// Positions per split: the plan's; with a device position the positions spread over the
+// planned splits.
+__device__ __forceinline__ int mla_f32_split_tokens(const MlaMK& p, int seq) {
+    if (!p.pos_dev) return p.split_tokens;
+    const int steps = (seq + kFStep - 1) / kFStep;
+    return (steps + p.splits - 1) / p.splits * kFStep;
+}
+
+template <int KL, int KR>
+__global__ void __launch_bounds__(kFWaves * 64, 1) mla_f32_kernel(const MlaMK p) {
+    using Gm = MlaF32Geom<KL, KR>;
+    constexpr int W = Gm::W, NJ = Gm::NJ, NV = Gm::NV, NG = Gm::NG, NJQ = Gm::NJQ;
+    constexpr int NR = NJ - NJQ > 0 ? NJ - NJQ : 1;
+    __shared__ __attribute__((aligned(1024))) char lds_v[kFWaves][Gm::VB];
+    __shared__ __attribute__((aligned(256))) char lds_q[kFHeads * Gm::QP];
+    __shared__ float sm_m[kFWaves][kFHeads], sm_l[kFWaves][kFHeads];
+
+    // as the 16-bit kernel: the head groups of one split run on one XCD
+    const int idx = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
+    if (idx >= p.groups * p.splits) return;
+    const int hg = idx % p.groups;
+    const int split = idx / p.groups;
+    const int seq = device_seq(p.pos_dev, p.seq_len);
+    const int split_tokens = mla_f32_split_tokens(p, seq);
+    const int nsplit = (seq + split_tokens - 1) / split_tokens;
+    if (split >= nsplit) return;
+    const int t_begin = split * split_tokens;
+    const int t_end = min(seq, t_begin + split_tokens);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & (kFWaves - 1);
+    const int q4 = lane >> 4;
+    const int l16 = lane & 15;
+    const int t_wave = t_begin + kFTile * wave;
+    const int nt = t_end > t_wave ? (t_end - t_wave + kFStep - 1) / kFStep : 0;
+
+    // ---- q~ of the workgroup's heads (padding heads repeat the last one and are not stored):
+    // loads issued before the tile's, so that waiting for them leaves the tile in flight
+    auto q_at = [&](int n, int c) __attribute__((always_inline)) {  // dims 4c .. 4c + 3 of head n
+        const size_t head = min(hg * kFHeads + n, p.heads - 1);
+        return *reinterpret_cast<const f32x4_t*>(4 * c < KL ? p.q_tilde + head * KL + 4 * c
+                                                            : p.q_rope + head * KR + (4 * c - KL));
+    };
+    constexpr int CQ = Gm::QL / 4;                       // staged chunks per head
+    constexpr int SQ = kFHeads * CQ / (kFWaves * 64);    // per thread
+    static_assert(SQ * kFWaves * 64 == kFHeads * CQ, "whole rounds of staging");
+    f32x4_t st[SQ];
+#pragma unroll
+    for (int i = 0; i < SQ; ++i) {
+        const int k = threadIdx.x + i * kFWaves * 64;
+        st[i] = q_at(k / CQ, k % CQ);
+    }
+    f32x4_t qr[NR];
+#pragma unroll
+    for (int j = 0; j < NJ - NJQ; ++j) qr[j] = q_at(l16, 4 * (NJQ + j) + q4);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // rows past the split's end lie outside the buffer range and read as zeros
+    f32x4_t kr[NJ];
+    const uint32_t voff = static_cast<uint32_t>(l16 * W * 4 + 16 * q4);
+    auto load_tile = [&](int i) __attribute__((always_inline)) {
+        const int t0 = t_wave + kFStep * i;
+        const long long phys = __builtin_amdgcn_readfirstlane(p.page_table[t0 >> kPageShift]);
+        const char* base = p.pool + (phys * kPageTokens + (t0 & (kPageTokens - 1))) * W * 4;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<char*>(base), 0, min(kFTile, t_end - t0) * W * 4, kBufferFlags);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            kr[j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, voff + 64 * j, 0, 0));
+    };
+    if (nt > 0) load_tile(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < SQ; ++i) {
+        const int k = threadIdx.x + i * kFWaves * 64;
+        const int n = k / CQ, c = k % CQ;
+        *reinterpret_cast<f32x4_t*>(lds_q + n * Gm::QP + 16 * (c ^ n)) = st[i] * p.qscale;
+    }
+#pragma unroll
+    for (int j = 0; j < NJ - NJQ; ++j) qr[j] *= p.qscale;
+    lds_barrier();
+    // chunk 4j + q4 of row l16 sits at 16 (j / 4) + ((4 (j % 4) + q4) ^ l16)
+    int cx[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cx[i] = 16 * ((4 * i + q4) ^ l16);
+
+    f32x4_t acc[NG][4];
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[g][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    char* const vt = lds_v[wave];
+
+    for (int i = 0; i < nt; ++i) {
+        // ---- scores: four chains (one per element of the 16-byte operands)
+        f32x4_t sc[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            f32x4_t qv;
+            if (j < NJQ) qv = *reinterpret_cast<const f32x4_t*>(lds_q + l16 * Gm::QP + cx[j & 3] + 256 * (j >> 2));
+            else qv = qr[j < NJQ ? 0 : j - NJQ];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[j][e], qv[e], sc[e], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            *reinterpret_cast<f32x4_t*>(vt + l16 * KL * 4 + cx[j & 3] + 256 * (j >> 2)) = kr[j];
+        if (i + 1 < nt) load_tile(i + 1);
+        __builtin_amdgcn_sched_barrier(0);  // the next tile's loads leave before the softmax
+
+        // ---- softmax: this lane's positions are t0 + 4q4 + r (lazy rescale, as above)
+        const int t0 = t_wave + kFStep * i;
+        float s[4];
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = t0 + 4 * q4 + r < t_end ? (sc[0][r] + sc[1][r]) + (sc[2][r] + sc[3][r]) : -INFINITY;
+            tmax = fmaxf(tmax, s[r]);
+        }
+        tmax = max_xor32(max_xor16(tmax));
+        const bool grow = tmax > m + kRescaleSlack;
+        const bool rescale = grow && m != -INFINITY;
+        if (__builtin_amdgcn_ballot_w64(rescale)) {
+            const float corr = rescale ? fast_exp2(m - tmax) : 1.f;
+            l *= corr;
+#pragma unroll
+            for (int g = 0; g < NG; ++g)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[g][e] *= corr;
+        }
+        if (grow) m = tmax;
+        const float mref = m == -INFINITY ? 0.f : m;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = fast_exp2(s[r] - mref);
+            l += s[r];
+        }
+
+        // ---- latent sum
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 4 * q4 + r;
+            const char* vr = vt + row * KL * 4 + 16 * (l16 ^ row);
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                const f32x4_t a = *reinterpret_cast<const f32x4_t*>(vr + 256 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[g][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], s[r], acc[g][e], 0, 0, 0);
+            }
+        }
+    }
+
+    // ---- the four waves merge through LDS: lane (q4, l16) holds dims 64g + 16q4 + 4r + e of
+    // head l16 in acc[g][e][r]
+    l = sum_xor32(sum_xor16(l));
+    if (q4 == 0) {
+        sm_m[wave][l16] = m;
+        sm_l[wave][l16] = l;
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<f32x4_t*>(vt + 16 * (64 * (4 * g + r) + lane)) =
+                f32x4_t{acc[g][0][r], acc[g][1][r], acc[g][2][r], acc[g][3][r]};
+    __syncthreads();
+    const int head = hg * kFHeads + l16;
+    if (head >= p.heads) return;
+    float M = -INFINITY, L = 0.f, c[kFWaves];
+#pragma unroll
+    for (int w = 0; w < kFWaves; ++w) M = fmaxf(M, sm_m[w][l16]);
+#pragma unroll
+    for (int w = 0; w < kFWaves; ++w) {
+        c[w] = sm_m[w][l16] == -INFINITY ? 0.f : fast_exp2(sm_m[w][l16] - M);
+        L = fmaf(sm_l[w][l16], c[w], L);
+    }
+    const size_t slot = static_cast<size_t>(head) * p.splits + split;
+#pragma unroll
+    for (int g = wave; g < NG; g += kFWaves)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < kFWaves; ++w)
+                o += c[w] * *reinterpret_cast<const f32x4_t*>(lds_v[w] + 16 * (64 * (4 * g + r) + lane));
+            const int d = 64 * g + 16 * q4 + 4 * r;
+            if (nsplit == 1) {
+                float* u = p.u + static_cast<size_t>(head) * KL + d;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) u[e] = o[e] / L;
+            } else {
+                *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.part_u) + slot * KL + d) = o;
+            }
+        }
+    if (nsplit > 1 && wave == 0 && q4 == 0) p.part_ml[slot] = make_float2(M, L);
+}
+
+// Split merge of the fp32 path: one workgroup per (head, 128-dim block); thread (grp, c4)
+// owns 4 dims and splits grp, grp + 8, ..., 8 of them loaded at once; the 8 groups merge
+// through LDS.
+template <int KL>
+__global__ void __launch_bounds__(256) mla_combine_f32_kernel(const MlaMK p) {
+    const int seq = device_seq(p.pos_dev, p.seq_len);
+    const int split_tokens = mla_f32_split_tokens(p, seq);
+    const int nsplit = (seq + split_tokens - 1) / split_tokens;
+    if (nsplit == 1) return;  // the split kernel wrote u
+    const int h = blockIdx.x;
+    const int c4 = threadIdx.x & 31;
+    const int grp = threadIdx.x >> 5;
+    const size_t base = static_cast<size_t>(h) * p.splits;
+    const f32x4_t* part = reinterpret_cast<const f32x4_t*>(static_cast<const float*>(p.part_u) + blockIdx.y * 128) + c4;
+    float m = -INFINITY, l = 0.f;
+    f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+    constexpr int kB = 8;
+    for (int s0 = grp; s0 < nsplit; s0 += 8 * kB) {
+        f32x4_t a[kB];
+        float2 ml[kB];
+#pragma unroll
+        for (int i = 0; i < kB; ++i) {
+            const int s = min(s0 + 8 * i, nsplit - 1);
+            a[i] = part[(base + s) * (KL / 4)];
+            ml[i] = p.part_ml[base + s];
+        }
+        float mb = m;
+#pragma unroll
+        for (int i = 0; i < kB; ++i) {
+            if (s0 + 8 * i >= nsplit) ml[i] = make_float2(-INFINITY, 0.f);  // a repeated split
+            mb = fmaxf(mb, ml[i].x);
+        }
+        const float cm = m == -INFINITY ? 0.f : fast_exp2(m - mb);
+        l *= cm;
+        o *= cm;
+#pragma unroll
+        for (int i = 0; i < kB; ++i) {
+            const float w = ml[i].x == -INFINITY ? 0.f : fast_exp2(ml[i].x - mb);
+            l = fmaf(ml[i].y, w, l);
+            if (s0 + 8 * i < nsplit) o += a[i] * w;
+        }
+        m = mb;
+    }
+    __shared__ float rm[256], rl[256];
+    __shared__ f32x4_t ro[256];
+    rm[threadIdx.x] = m;
+    rl[threadIdx.x] = l;
+    ro[threadIdx.x] = o;
+    __syncthreads();
+    if (threadIdx.x < 128) {  // dim e of column cc
+        const int cc = threadIdx.x >> 2, e = threadIdx.x & 3;
+        float M = -INFINITY, L = 0.f, t = 0.f;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) M = fmaxf(M, rm[g * 32 + cc]);
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const float c = rm[g * 32 + cc] == -INFINITY ? 0.f : fast_exp2(rm[g * 32 + cc] - M);
+            L = fmaf(rl[g * 32 + cc], c, L);
+            t = fmaf(reinterpret_cast<const float*>(ro)[4 * (g * 32 + cc) + e], c, t);
+        }
+        p.u[static_cast<size_t>(h) * KL + blockIdx.y * 128 + threadIdx.x] = t / L;
+    }
+}
+
 bool mfma_eligible(const MlaArgs& a) {
     return a.dtype != QR_DTYPE_F32 && a.kv_lora == kMfmaLora && (a.rope == 0 || a.rope == 64);
+}
+
+// fp32 latents whose width is made of the fp32 kernel's tiles.
+bool f32_eligible(const MlaArgs& a) {
+    return a.dtype == QR_DTYPE_F32 && (a.kv_lora == 256 || a.kv_lora == 512) &&
+           (a.rope == 0 || a.rope == 32 || a.rope == 64);
 }
 
 int cus() {
@@ -796,6 +1111,13 @@ MlaPlan plan_mla(const MlaArgs& a) {
         pl.split_tokens = tiles_per_split * kMTile;
         // room for 16-byte aligned copies of q~ / q_rope when the caller's are not
         q_copy = align256(static_cast<size_t>(a.heads) * a.kv_lora * 4) + align256(static_cast<size_t>(a.heads) * a.rope * 4);
+    } else if (f32_eligible(a)) {
+        // about one workgroup per CU: (16-head group) x split, splits of whole 64-position steps
+        const int groups = (a.heads + kFHeads - 1) / kFHeads;
+        const int steps = (a.seq_len + kFStep - 1) / kFStep;
+        const int want = std::min(std::max(1, cus() / groups), steps);
+        pl.split_tokens = (steps + want - 1) / want * kFStep;
+        q_copy = align256(static_cast<size_t>(a.heads) * a.kv_lora * 4) + align256(static_cast<size_t>(a.heads) * a.rope * 4);
     } else {
         pl.split_tokens = kGenericSplit;
     }
@@ -812,6 +1134,30 @@ namespace {
 template <bool SRC_BF16, int KR>
 hipError_t launch_tile(const MlaMK& k, hipStream_t stream) {
     hipLaunchKernelGGL((mla_tile_kernel<SRC_BF16, KR>), dim3(8 * k.per_xcd), dim3(kMWaves * 64), 0, stream, k);
+    return hipGetLastError();
+}
+// The tile kernels read q~ and q_rope as float4: 16-byte aligned, or copied to `room`.
+hipError_t aligned_q(const MlaArgs& a, char* room, hipStream_t stream, const float** q_tilde, const float** q_rope) {
+    *q_tilde = a.q_tilde;
+    *q_rope = a.q_rope;
+    if (((reinterpret_cast<uintptr_t>(a.q_tilde) | reinterpret_cast<uintptr_t>(a.q_rope)) & 15) == 0) return hipSuccess;
+    const size_t bytes = static_cast<size_t>(a.heads) * a.kv_lora * 4;
+    float* qt = reinterpret_cast<float*>(room);
+    float* qr = reinterpret_cast<float*>(room + align256(bytes));
+    hipError_t e = hipMemcpyAsync(qt, a.q_tilde, bytes, hipMemcpyDeviceToDevice, stream);
+    if (e == hipSuccess && a.rope)
+        e = hipMemcpyAsync(qr, a.q_rope, static_cast<size_t>(a.heads) * a.rope * 4, hipMemcpyDeviceToDevice, stream);
+    *q_tilde = qt;
+    *q_rope = a.rope ? qr : nullptr;
+    return e;
+}
+
+template <int KL, int KR>
+hipError_t launch_f32(const MlaMK& k, hipStream_t stream) {
+    hipLaunchKernelGGL((mla_f32_kernel<KL, KR>), dim3(8 * k.per_xcd), dim3(kFWaves * 64), 0, stream, k);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || k.splits == 1) return e;
+    hipLaunchKernelGGL((mla_combine_f32_kernel<KL>), dim3(k.heads, KL / 128), dim3(256), 0, stream, k);
     return hipGetLastError();
 }
 }  // namespace
@@ -836,28 +1182,36 @@ hipError_t launch_mla(const MlaArgs& a, const MlaPlan& pl, void* workspace, hipS
         k.part_u = ws;
         k.part_ml = reinterpret_cast<float2*>(ws + align256(slots * a.kv_lora * 2));
         k.part_e = reinterpret_cast<signed char*>(ws + align256(slots * a.kv_lora * 2) + align256(slots * 8));
-        // the kernel reads q~ / q_rope as float4
-        k.q_tilde = a.q_tilde;
-        k.q_rope = a.q_rope;
-        const bool misaligned = (reinterpret_cast<uintptr_t>(a.q_tilde) | reinterpret_cast<uintptr_t>(a.q_rope)) & 15;
-        if (misaligned) {
-            float* qt = reinterpret_cast<float*>(ws + part_bytes);
-            float* qr = reinterpret_cast<float*>(ws + part_bytes + align256(static_cast<size_t>(a.heads) * a.kv_lora * 4));
-            hipError_t e = hipMemcpyAsync(qt, a.q_tilde, static_cast<size_t>(a.heads) * a.kv_lora * 4, hipMemcpyDeviceToDevice, stream);
-            if (e == hipSuccess && a.rope)
-                e = hipMemcpyAsync(qr, a.q_rope, static_cast<size_t>(a.heads) * a.rope * 4, hipMemcpyDeviceToDevice, stream);
-            if (e != hipSuccess) return e;
-            k.q_tilde = qt;
-            k.q_rope = a.rope ? qr : nullptr;
-        }
+        hipError_t e = aligned_q(a, ws + part_bytes, stream, &k.q_tilde, &k.q_rope);
+        if (e != hipSuccess) return e;
         k.qscale = static_cast<float>(static_cast<double>(a.scale) * 1.4426950408889634);
-        hipError_t e;
         const bool bf = a.dtype == QR_DTYPE_BF16;
         if (a.rope) e = bf ? launch_tile<true, 64>(k, stream) : launch_tile<false, 64>(k, stream);
         else e = bf ? launch_tile<true, 0>(k, stream) : launch_tile<false, 0>(k, stream);
         if (e != hipSuccess || pl.splits == 1) return e;
         hipLaunchKernelGGL(mla_combine_wide_kernel, dim3(a.heads, kMfmaLora / 64), dim3(256), 0, stream, k);
         return hipGetLastError();
+    }
+    if (f32_eligible(a)) {
+        MlaMK k{};
+        k.pool = static_cast<const char*>(a.pool);
+        k.page_table = a.page_table;
+        k.heads = a.heads;
+        k.seq_len = a.seq_len;
+        k.pos_dev = a.pos_dev;
+        k.split_tokens = pl.split_tokens;
+        k.splits = pl.splits;
+        k.groups = (a.heads + kFHeads - 1) / kFHeads;
+        k.per_xcd = (k.groups * pl.splits + 7) / 8;
+        k.u = a.u;
+        const size_t part_bytes = pl.splits > 1 ? align256(slots * a.kv_lora * 4) + align256(slots * 8) : 0;
+        k.part_u = ws;
+        k.part_ml = reinterpret_cast<float2*>(ws + align256(slots * a.kv_lora * 4));
+        const hipError_t e = aligned_q(a, ws + part_bytes, stream, &k.q_tilde, &k.q_rope);
+        if (e != hipSuccess) return e;
+        k.qscale = static_cast<float>(static_cast<double>(a.scale) * 1.4426950408889634);
+        if (a.kv_lora == 512) return a.rope == 64 ? launch_f32<512, 64>(k, stream) : a.rope == 32 ? launch_f32<512, 32>(k, stream) : launch_f32<512, 0>(k, stream);
+        return a.rope == 64 ? launch_f32<256, 64>(k, stream) : a.rope == 32 ? launch_f32<256, 32>(k, stream) : launch_f32<256, 0>(k, stream);
     }
     MlaK k{};
     k.pool = static_cast<const char*>(a.pool);

@@ -67,6 +67,42 @@ def test_mla_fp32_generic(gpu, heads, kv_lora, rope, n):
     check_mla(got, lat, qt, qrp, kv_lora, rope, s, 1e-4, f"f32 H{heads} lora{kv_lora} rope{rope} n{n}")
 
 
+@pytest.mark.parametrize("heads,kv_lora,rope,n,pos", [
+    (1, 512, 64, 1, 0),          # one position, one head of a 16-head group
+    (17, 512, 64, 15, None),     # one head past a group; less than one 16-position tile
+    (16, 512, 0, 64, None),      # exactly one step of four tiles
+    (20, 512, 32, 65, None),     # one position past a step
+    (128, 512, 64, 300, 256),    # across a page; rows past pos resident
+    (33, 256, 64, 2000, None),
+    (128, 256, 32, 4099, None),  # every split, the last of them ragged
+    (5, 256, 0, 777, 130),
+])
+def test_mla_fp32_tiles(gpu, heads, kv_lora, rope, n, pos):
+    """fp32 tile kernel against the oracle and fp64.  A score is a chain of kv_lora + rope fp32
+    products of N(0,1) values, |s| <= about 12: its rounding error is at most ~12 sqrt(576) 2^-24
+    = 1.7e-5 and moves each weight, and so u, by no more than that: 2e-5 rel-L2."""
+    import torch
+
+    got, lat, qt, qrp, s = run_mla("f32", heads, kv_lora, rope, n, pos=pos, seed=heads + n)
+    check_mla(got, lat, qt, qrp, kv_lora, rope, s, 1e-4, f"f32 H{heads} lora{kv_lora} rope{rope} n{n}")
+    want = oracle.mla_attention_f64(lat, qt, qrp, kv_lora, rope, s)
+    assert errors(got, want)[1] <= 2e-5
+    # the position read on the device (splits planned for max_seq), q rows 4-byte aligned only
+    def odd(a):
+        t = torch.zeros(a.size + 1, device=gpu)
+        t[1:] = torch.from_numpy(np.ascontiguousarray(a).reshape(-1))
+        return t[1:]
+    p = len(lat) - 1
+    with qr.MlaLatentCache(1, kv_lora + rope, n + 1000, rope=rope) as m:
+        m.AppendRange(0, 0, lat)
+        u = torch.full((heads * kv_lora + 1,), 7.0, device=gpu)
+        m.AbsorbedAttentionStepDev(0, torch.tensor([p], dtype=torch.int32, device=gpu), odd(qt),
+                                   odd(qrp) if rope else None, u[:-1], s)
+        torch.cuda.synchronize()
+        assert errors(u[:-1].cpu().numpy().reshape(heads, kv_lora), want)[1] <= 2e-5
+        assert u[-1].item() == 7.0
+
+
 @pytest.mark.parametrize("rope", [0, 16])
 def test_mla_absorbed_equals_expanded_through_gpu(gpu, rope):
     """Cli/Commands.cs:2065-2152: q-absorb -> GPU latent attention -> W_UV equals the
