@@ -511,7 +511,8 @@ int chunk_common(qr_kv* kv, int seq_id, int layer, int pos0, int nq, const void*
     }
     float* q32 = reinterpret_cast<float*>(st + ((qbytes + 255) & ~size_t(255)));
     float* dout = out_is_dev ? attn : q32 + nq * rowf;
-    if (chunk_mfma_eligible(kv->dtype, kv->head_dim, kv->heads, kv->kv_heads)) {
+    const bool tiles16 = chunk_mfma_eligible(kv->dtype, kv->head_dim, kv->heads, kv->kv_heads);
+    if (tiles16 || chunk_f32_eligible(kv->dtype, kv->head_dim, kv->heads, kv->kv_heads, pos0, nq)) {
         // MFMA tiles read each K/V tile once for a block of queries
         ChunkArgs c{};
         c.pool = kv->store.pool();
@@ -525,11 +526,12 @@ int chunk_common(qr_kv* kv, int seq_id, int layer, int pos0, int nq, const void*
         c.q_dtype = q_dtype;
         c.out = dout;
         c.scale = scale;
-        const ChunkPlan plan = plan_chunk(c);
+        const ChunkPlan plan = tiles16 ? plan_chunk(c) : plan_chunk_f32(c);
         QR_TRY(grow_workspace(kv, plan.workspace_bytes, stream));
-        QR_HIP(launch_chunk(c, plan, kv->workspace.get(), stream, kv->split_event));
+        QR_HIP(tiles16 ? launch_chunk(c, plan, kv->workspace.get(), stream, kv->split_event)
+                       : launch_chunk_f32(c, plan, kv->workspace.get(), stream, kv->split_event));
     } else {
-        // exact fp32 path: every query is one decode entry with its causal length; the
+        // other shapes: every query is one decode entry with its causal length; the
         // decode kernels read fp32 queries, so 16-bit ones are widened first (the MFMA
         // branch above reads them in their own type)
         const float* qf = static_cast<const float*>(qsrc);

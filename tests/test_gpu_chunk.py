@@ -128,3 +128,67 @@ def test_chunk_mfma_shapes(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dtype):
     for i in sorted({0, nq // 2, nq - 1}):
         check_query(out[i], Kd[:pos0 + i + 1], Vd[:pos0 + i + 1], qd[i], heads, kv_heads, D, scale,
                     TOL_REL[dtype], f"{dtype} H{heads}/Hkv{kv_heads}/D{D} pos0 {pos0} query {i}")
+
+
+def causal_f64(K, V, q, heads, kv_heads, D, pos0, scale):
+    """All queries of a chunk in float64."""
+    K, V, q = (np.asarray(x, np.float64) for x in (K, V, q))
+    out = np.empty((q.shape[0], heads * D))
+    seen = np.arange(K.shape[0])[None, :] <= pos0 + np.arange(q.shape[0])[:, None]
+    for h in range(heads):
+        j = slice(h * kv_heads // heads * D, (h * kv_heads // heads + 1) * D)
+        s = np.where(seen, q[:, h * D:(h + 1) * D] @ K[:, j].T * scale, -np.inf)
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, h * D:(h + 1) * D] = p @ V[:, j] / p.sum(1, keepdims=True)
+    return out
+
+
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq,q_dtype", [
+    ("f32", 32, 8, 96, 0, 2, "f32"),         # 8 rows per kv head: the fewest, one tile of 2 keys
+    ("f32", 32, 8, 96, 33, 8, "f32"),        # 32 rows, two position halves, second tile of 9 keys
+    ("f32", 32, 8, 64, 0, 65, "f32"),        # the fewest queries that need no key bytes
+    ("f32", 32, 8, 128, 5000, 9, "f32"),     # 36 rows, keys split
+    ("f32", 32, 8, 128, 0, 333, "f32"),      # from scratch: every tile masked for some block
+    ("f32", 28, 4, 128, 255, 75, "bf16"),    # group 7, 16-bit queries, crosses a page
+    ("f32", 24, 8, 96, 1000, 200, "f32"),    # group 3, head_dim 96 (8-byte V reads)
+    ("f32", 16, 16, 256, 300, 67, "f16"),    # group 1, head_dim 256
+    ("f32", 64, 1, 64, 7, 66, "f32"),        # 64 heads on one kv head
+    ("f32", 32, 8, 64, 700, 600, "f32"),     # two N tiles
+    ("f16", 24, 8, 96, 500, 130, "f16"),     # 16-bit pages, token-major
+    ("bf16", 32, 8, 96, 90, 40, "f32"),
+    ("bf16", 64, 8, 256, 250, 70, "bf16"),
+    ("f16", 8, 2, 256, 9000, 7, "f32"),
+    ("f32", 32, 8, 128, 3000, 5, "f32"),     # 20 rows over split keys, from the byte line up
+])
+def test_chunk_f32_tiles(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dtype):
+    """fp32 arithmetic over the exactly decoded cache: fp32 sums over up to 5,000 keys, 5e-6
+    relative (2^-24 times the square root of the terms, over the cancellation of the sum)."""
+    n = pos0 + nq
+    Kb, Kd, Vb, Vd = make(n + heads, n, kv_heads * D, dtype)
+    qb, qd = to_dtype_bits(np.random.default_rng(n).standard_normal((nq, heads * D), dtype=np.float32), q_dtype)
+    scale = 1 / math.sqrt(D)
+    with qr.PagedKvCache(1, heads, kv_heads, D, n + 10, kv_dtype=dtype) as kv:
+        kv.AppendRange(0, 0, Kb, Vb, src_dtype=dtype)
+        out = kv.AttentionChunk(0, pos0, qb, scale, q_dtype=q_dtype)
+    want = causal_f64(Kd, Vd, qd, heads, kv_heads, D, pos0, scale)
+    for i in range(nq):
+        a, r = errors(out[i], want[i])
+        assert r <= 5e-6, f"query {i}: rel-L2 {r:.2e} max-abs {a:.2e}"
+
+
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,nq", [("f32", 8, 2, 64, 70), ("f32", 8, 2, 128, 100), ("bf16", 8, 4, 96, 40),
+                                                         ("f16", 8, 8, 256, 75)])
+def test_chunk_f32_tiles_unseen_infinities(gpu, dtype, heads, kv_heads, D, nq):
+    """An infinite V reaches the queries that see its position and no other."""
+    Kb, Kd, Vb, Vd = make(3, nq, kv_heads * D, dtype)
+    bad = nq - 2
+    Vi, _ = to_dtype_bits(np.where(np.arange(nq)[:, None] == bad, np.float32(np.inf), Vd), dtype)
+    q = np.random.default_rng(4).standard_normal((nq, heads * D), dtype=np.float32)
+    out = {}
+    for name, v in (("plain", Vb), ("inf", Vi)):
+        with qr.PagedKvCache(1, heads, kv_heads, D, nq, kv_dtype=dtype) as kv:
+            kv.AppendRange(0, 0, Kb, v, src_dtype=dtype)
+            out[name] = kv.AttentionChunk(0, 0, q, 1 / math.sqrt(D))
+    for i in range(bad):
+        assert errors(out["inf"][i], out["plain"][i])[1] <= 5e-6, i
+    assert np.all(out["inf"][bad:] == np.inf)
