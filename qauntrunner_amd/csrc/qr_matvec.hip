@@ -11,13 +11,15 @@
 //   Q6_K          per block: 256 products summed in (half, l, q1..q4) order; sum += d*dot
 // Every product and sum is separately rounded (mul_rn / add_rn / sub_rn).
 //
-// Kernels (every weight byte is read once per input vector):
+// Kernels (every weight byte is read once per input vector, or once per up to four of them):
 //   matvec_blk_persistent  Q4_K: x in registers per 64-column item, row tiles double
 //                          buffered in registers, block terms per thread, in-order sums last
 //   matvec_blk_ring        Q8_0: the same items with row tiles streamed through an LDS ring
-//   matvec_fp_wave         F32/F16/BF16: one wave per 8 rows, lane = (row, DotF32 lane),
+//   matvec_blk_multi       two and more vectors of Q8_0, Q4_0 and Q4_K, one of Q4_0: x of up to
+//                          four vectors in registers per 32-column item
+//   matvec_fp_wave         F32/F16/BF16: one wave per 8 rows (and up to four vectors), lane = (row, DotF32 lane),
 //                          1 KiB row segments through an LDS ring
-//   matvec_kernel          everything else (Q4_0, Q6_K, unaligned rows): LDS tiles of R rows,
+//   matvec_kernel          everything else (Q6_K, rows of odd items): LDS tiles of R rows,
 //                          block terms in parallel, one thread per row adds them in order
 #include <algorithm>
 
@@ -378,11 +380,11 @@ struct BlkGroup {
     float* y[kMatVecGroupMax];
 };
 
-__device__ __forceinline__ int group_member(int n, const int (&start)[kMatVecGroupMax + 1]) {
+__device__ __forceinline__ int group_member(int n, const int (&start)[kMatVecGroupMax + 1], int wg) {
     int m = 0;
 #pragma unroll
     for (int i = 1; i < kMatVecGroupMax; ++i)
-        if (i < n && static_cast<int>(blockIdx.x) >= start[i]) m = i;
+        if (i < n && wg >= start[i]) m = i;
     return m;
 }
 
@@ -507,7 +509,7 @@ __global__ __launch_bounds__(512) void matvec_blk_persistent(MatVecArgs a, MvBlk
     typedef typename PolLoad<Pol>::type V;
     extern __shared__ __align__(16) uint8_t mv_lds[];
     float* terms = reinterpret_cast<float*>(mv_lds);
-    const int mg = group_member(gr.n, gr.start);  // this workgroup's matrix (uniform)
+    const int mg = group_member(gr.n, gr.start, blockIdx.x);  // this workgroup's matrix (uniform)
     a.w = gr.w[mg];
     a.rows = gr.rows[mg];
     a.y = gr.y[mg];
@@ -619,7 +621,7 @@ __global__ __launch_bounds__(256) void matvec_blk_ring(MatVecArgs a, MvRing k, B
     typedef typename PolLoad<Pol>::type V;
     extern __shared__ __align__(1024) char ring_lds[];
     float* terms = reinterpret_cast<float*>(ring_lds + kRingSlots * k.slot_bytes);
-    const int mg = group_member(gr.n, gr.start);  // this workgroup's matrix (uniform)
+    const int mg = group_member(gr.n, gr.start, blockIdx.x);  // this workgroup's matrix (uniform)
     a.w = gr.w[mg];
     a.rows = gr.rows[mg];
     a.y = gr.y[mg];
@@ -685,6 +687,259 @@ __global__ __launch_bounds__(256) void matvec_blk_ring(MatVecArgs a, MvRing k, B
     }
 }
 
+// ---- several input vectors (nq >= 2), block formats: Q8_0, Q4_0 and Q4_K with items of 32
+// columns (a Q8_0 or Q4_0 block, a Q4_K sub-block; one term each).
+//
+// One vector per workgroup row (grid y), the form before, read and decoded the weights once per
+// vector: the 8 vectors of a verify over the seven Q8_0 matrices of an 8B layer took 383 us, at
+// 4.9 TB/s from the memory-side cache.  Here a thread keeps the 32 x values of its item for NV
+// vectors in registers (NV <= 4: 128 registers) and multiplies every weight it decodes with all
+// of them, so the weights are read ceil(nq / 4) times and a weight costs its decode once and a
+// multiply and an add (separately rounded) per vector: 165 us for those 8 vectors.  The bound is
+// then the VALU: 2 of the 2.4 instructions per weight and vector are those (107 us at one
+// instruction per 4 cycles and SIMD); gate and up run at 80% of it, the rest are the prologues
+// (x), the in-order sums and, at 14336 columns, seven waves per CU.  Q4_0 and Q4_K layers of 8
+// vectors: 807 -> 137 and 226 -> 148 us; one vector of Q4_0, 145 -> 50.
+//
+// Row tiles stream through two LDS slots by direct-to-LDS loads as in matvec_blk_ring; the
+// terms of all of a workgroup's rows stay in LDS and are summed in order at the end.
+//
+// A chain that starts at its first product instead of +0 + product can differ only in the sign
+// of a zero term, and y's own chain starts at +0, which no added zero changes.
+__device__ __forceinline__ float hsum8_from_first(const float (&v)[8]) {
+    float s = v[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) s = add_rn(s, v[i]);
+    return s;
+}
+__device__ __forceinline__ float ubyte_f32(uint32_t w, int k) { return static_cast<float>((w >> (8 * k)) & 0xFFu); }
+
+// Policies: kDw dwords of an item (read from its row in LDS), decoded to 32 weights q and
+// scales; prep: the x-only sum that the term needs; term: one vector's term.
+struct MulQ8 {
+    static constexpr int kDw = 9, kAlign = 4, kItemBytes = 34;
+    struct Scale { float d; };
+    __device__ static void load(const char* row, int pc, uint32_t (&w)[kDw]) {
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(row + ((34 * pc) & ~3));
+#pragma unroll
+        for (int i = 0; i < kDw; ++i) w[i] = p[i];
+    }
+    __device__ static void decode(const uint32_t (&w)[kDw], int pc, float (&q)[32], Scale& s) {
+        const bool odd = pc & 1;  // odd blocks start in the middle of a dword
+        s.d = f16_bits_to_f32(static_cast<uint16_t>(odd ? w[0] >> 16 : w[0] & 0xFFFFu));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t v = odd ? w[i + 1] : (w[i] >> 16) | (w[i + 1] << 16);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[4 * i + k] = static_cast<float>(static_cast<int8_t>((v >> (8 * k)) & 0xFFu));
+        }
+    }
+    __device__ static float prep(const float (&)[32]) { return 0.0f; }
+    __device__ static float term(const float (&q)[32], const Scale& s, const float (&x)[32], float) {
+        float acc[8];
+#pragma unroll
+        for (int L = 0; L < 8; ++L) {
+            acc[L] = mul_rn(q[L], x[L]);
+#pragma unroll
+            for (int k = 1; k < 4; ++k) acc[L] = add_rn(acc[L], mul_rn(q[8 * k + L], x[8 * k + L]));
+        }
+        return mul_rn(s.d, hsum8_from_first(acc));
+    }
+};
+
+struct MulQ40 {
+    static constexpr int kDw = 5, kAlign = 4, kItemBytes = 20;
+    struct Scale { float d; };
+    __device__ static void load(const char* row, int pc, uint32_t (&w)[kDw]) {
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(row + 20 * pc);
+#pragma unroll
+        for (int i = 0; i < kDw; ++i) w[i] = p[i];
+    }
+    __device__ static void decode(const uint32_t (&w)[kDw], int, float (&q)[32], Scale& s) {
+        s.d = f16_bits_to_f32(static_cast<uint16_t>(w[0] & 0xFFFFu));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // bytes 4i .. 4i + 3 of the 16
+            const uint32_t v = (w[i] >> 16) | (w[i + 1] << 16);
+            const uint32_t lo = nibble_mask(v), hi = nibble_mask(v >> 4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                q[4 * i + k] = ubyte_f32(lo, k);
+                q[16 + 4 * i + k] = ubyte_f32(hi, k);
+            }
+        }
+    }
+    __device__ static float prep(const float (&x)[32]) {  // HSum of the x lanes (DotKernels.cs:134-178)
+        float ax[8];
+#pragma unroll
+        for (int l = 0; l < 8; ++l) ax[l] = add_rn(add_rn(add_rn(add_rn(0.0f, x[l]), x[8 + l]), x[16 + l]), x[24 + l]);
+        return hsum8(ax);
+    }
+    __device__ static float term(const float (&q)[32], const Scale& s, const float (&x)[32], float sum_x) {
+        float acc[8];
+#pragma unroll
+        for (int L = 0; L < 8; ++L) {
+            acc[L] = mul_rn(q[L], x[L]);
+#pragma unroll
+            for (int k = 1; k < 4; ++k) acc[L] = add_rn(acc[L], mul_rn(q[8 * k + L], x[8 * k + L]));
+        }
+        return sub_rn(mul_rn(s.d, hsum8_from_first(acc)), mul_rn(mul_rn(8.0f, s.d), sum_x));
+    }
+};
+
+struct MulQ4K {
+    static constexpr int kDw = 12, kAlign = 16, kItemBytes = 18;
+    struct Scale { float a, mm; };
+    __device__ static void load(const char* row, int pc, uint32_t (&w)[kDw]) {
+        const char* b = row + (pc >> 3) * 144;
+        const u32x4_t h = *reinterpret_cast<const u32x4_t*>(b);
+        const u32x4_t q0 = *reinterpret_cast<const u32x4_t*>(b + 16 + 32 * ((pc >> 1) & 3));
+        const u32x4_t q1 = *reinterpret_cast<const u32x4_t*>(b + 32 + 32 * ((pc >> 1) & 3));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            w[i] = h[i];
+            w[4 + i] = q0[i];
+            w[8 + i] = q1[i];
+        }
+    }
+    __device__ static void decode(const uint32_t (&w)[kDw], int pc, float (&q)[32], Scale& s) {
+        const u32x4_t h = {w[0], w[1], w[2], w[3]};
+        int sc, m;
+        q4k_scale_min(h, (pc >> 1) & 3, pc & 1, sc, m);
+        s.a = mul_rn(f16_bits_to_f32(static_cast<uint16_t>(w[0] & 0xFFFFu)), static_cast<float>(sc));
+        s.mm = mul_rn(f16_bits_to_f32(static_cast<uint16_t>(w[0] >> 16)), static_cast<float>(m));
+        const uint32_t sh = 4u * static_cast<uint32_t>(pc & 1);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t v = nibble_mask(w[4 + i] >> sh);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[4 * i + k] = ubyte_f32(v, k);
+        }
+    }
+    __device__ static float prep(const float (&x)[32]) {  // SubSum, in order
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) s = add_rn(s, x[i]);
+        return s;
+    }
+    __device__ static float term(const float (&q)[32], const Scale& s, const float (&x)[32], float ss) {
+        float v[2];
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {  // VecDot16
+            float acc[8];
+#pragma unroll
+            for (int L = 0; L < 8; ++L)
+                acc[L] = add_rn(mul_rn(q[16 * half + L], x[16 * half + L]), mul_rn(q[16 * half + 8 + L], x[16 * half + 8 + L]));
+            v[half] = hsum8_from_first(acc);
+        }
+        return sub_rn(mul_rn(s.a, add_rn(v[0], v[1])), mul_rn(s.mm, ss));
+    }
+};
+
+struct MvMulti {
+    int P, tpg, R, tstride;
+    int passes;      // over the weights: ceil(nq / NV)
+    int flush;       // tiles whose terms LDS holds: their rows are summed together
+    int slot_bytes;  // of a tile in LDS
+};
+
+// LDS slots of the tile ring (three or four measured slower: fewer tiles' terms fit beside them,
+// so the in-order sums come more often)
+constexpr int kMulSlots = 2;
+// 1 KiB loads of a wave and tile: a wave's 64 items, at least one row's part of the tile
+template <class Pol> constexpr int kMulUnits = (64 * Pol::kItemBytes + 1023) / 1024;
+
+template <class Pol, int NV>
+__global__ __launch_bounds__(512) void matvec_blk_multi(MatVecArgs a, MvMulti k, BlkGroup gr) {
+    extern __shared__ __align__(1024) char ring_lds[];
+    constexpr int U = kMulUnits<Pol>;
+    float* terms = reinterpret_cast<float*>(ring_lds + kMulSlots * k.slot_bytes);
+    // Launch slot b runs on XCD b % 8: the passes over one set of rows are neighbours there, so
+    // that the second reads the weights that the first brought into the L2.
+    const int slot0 = static_cast<int>(blockIdx.x) >> 3;
+    const int wg = (slot0 / k.passes) * 8 + (static_cast<int>(blockIdx.x) & 7);
+    if (wg >= gr.start[gr.n]) return;
+    const int mg = group_member(gr.n, gr.start, wg);  // this workgroup's matrix (uniform)
+    a.w = gr.w[mg];
+    a.rows = gr.rows[mg];
+    a.y = gr.y[mg];
+    const int bx = wg - gr.start[mg];
+    const int G = gr.start[mg + 1] - gr.start[mg];
+    const int cnt = (gr.ntiles[mg] - bx + G - 1) / G;  // tiles of this workgroup, >= 1
+    const int t = threadIdx.x;
+    const int lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int waves = static_cast<int>(blockDim.x) >> 6;
+    const int g = min(t / k.tpg, k.R - 1);  // threads past the last row group store nothing
+    const bool active = t < k.R * k.tpg && t - g * k.tpg < k.P;
+    const int pc = min(t - g * k.tpg, k.P - 1);
+    const int q0 = slot0 % k.passes * NV;
+
+    // The workgroup's tile s, U loads a wave: bytes past the tile, the matrix or (s >= cnt) the
+    // last tile lie outside the resource and read as zeros.
+    auto dma = [&](int s) {
+        const int r0 = (bx + min(s, cnt - 1) * G) * k.R;
+        const int nrec = s < cnt ? min(k.R, static_cast<int>(a.rows) - r0) * static_cast<int>(a.row_bytes) : 0;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t*>(a.w + static_cast<long long>(r0) * a.row_bytes), static_cast<short>(0), nrec,
+            kBufferFlags);
+        char* slot = ring_lds + (s % kMulSlots) * k.slot_bytes;
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int u = wave + waves * i;
+            buffer_load_lds16(rs, slot + 1024 * u, static_cast<uint32_t>(16 * lane), static_cast<uint32_t>(1024 * u));
+        }
+    };
+    // x first, awaited before any DMA is in flight (see matvec_blk_ring); vectors past the last
+    // repeat it and are not stored
+    float x[NV][32], aux[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const float4* x4 =
+            reinterpret_cast<const float4*>(a.x + static_cast<long long>(min(q0 + v, a.nq - 1)) * a.cols + 32 * pc);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float4 f = x4[i];
+            x[v][4 * i] = f.x;
+            x[v][4 * i + 1] = f.y;
+            x[v][4 * i + 2] = f.z;
+            x[v][4 * i + 3] = f.w;
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) aux[v] = Pol::prep(x[v]);
+    wait_vmcnt<0>();
+#pragma unroll
+    for (int s = 0; s < kMulSlots - 1; ++s) dma(s);
+    for (int s = 0, held = 0; s < cnt; ++s) {
+        wait_vmcnt<(kMulSlots - 2) * U>();  // this wave's part of tile s has landed
+        lds_barrier();  // everyone's has, the slot filled next was read, the summed terms too
+        dma(s + kMulSlots - 1);
+        uint32_t w[Pol::kDw];
+        Pol::load(ring_lds + (s % kMulSlots) * k.slot_bytes + g * static_cast<int>(a.row_bytes), pc, w);
+        float q[32];
+        typename Pol::Scale sc;
+        Pol::decode(w, pc, q, sc);
+        float* out = terms + ((held * k.R + g) * NV) * k.tstride + pc;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const float term = Pol::term(q, sc, x[v], aux[v]);
+            if (active) out[v * k.tstride] = term;
+        }
+        if (++held < k.flush && s + 1 < cnt) continue;
+        // in-order sums of the held tiles' rows, one (row, vector) per thread
+        lds_barrier();
+        for (int i = t; i < held * k.R * NV; i += blockDim.x) {
+            const int sr = i / NV, v = i - sr * NV;
+            const int h = sr / k.R, r = sr - h * k.R;
+            const long long row = static_cast<long long>(bx + (s + 1 - held + h) * G) * k.R + r;
+            if (row >= a.rows || q0 + v >= a.nq) continue;
+            a.y[static_cast<long long>(q0 + v) * a.rows + row] = ordered_row_sum(terms + i * k.tstride, k.P);
+        }
+        held = 0;
+    }
+    wait_dma();
+}
+
 // ---- F32 / F16 / BF16 (DotF32 order, DotKernels.cs:52-100).  Row r's lane L accumulates
 // k = 8c + L over the chunks c in order, so every row is 8 serial chains.  A workgroup is one
 // wave and R <= 8 rows, lane 8r + L the chain (row r, lane L).  The wave streams its rows in segments of 1 KiB per row through a
@@ -698,26 +953,36 @@ __global__ __launch_bounds__(256) void matvec_blk_ring(MatVecArgs a, MvRing k, B
 constexpr int kFwSlots = 2;
 constexpr int kFwRowPad = 1024 + 16;  // LDS bytes per row segment: rows land on distinct banks
 
-template <int FMT, int R>
+// NV input vectors (1 to 4): a weight is read from LDS and decoded once for all of them, and
+// x segments of all NV sit in the slot.
+template <int FMT, int R, int NV>
 struct FwGeom {
     static constexpr int B = FMT == QR_FMT_F32 ? 32 : 16;     // bytes per chunk of 8 weights
     static constexpr int SEG = 1024 / B;                       // chunks per segment
     static constexpr int XBYTES = SEG * 32;                    // x bytes per segment
     static constexpr int XDMA = XBYTES / 1024;                 // DMAs of x per segment
-    static constexpr int SLOT = R * kFwRowPad + XBYTES;        // bytes per slot
-    static constexpr int DMAS = R + XDMA;                      // DMAs per segment
+    static constexpr int SLOT = R * kFwRowPad + NV * XBYTES;   // bytes per slot
+    static constexpr int DMAS = R + NV * XDMA;                 // DMAs per segment
 };
 
-// The product of the weight at p (LDS) and x.  F16: fma(w, x, +0) in one v_fma_mix_f32 (the
+template <int FMT> struct FwWeight { typedef float type; };
+template <> struct FwWeight<QR_FMT_F16> { typedef _Float16 type; };
+
+// The product of a weight and x.  F16: fma(w, x, +0) in one v_fma_mix_f32 (the
 // half converted exactly inside); it equals the rounded product w*x except that a -0 product
 // becomes +0, which no chain can tell apart: a lane sum starts at +0 and never becomes -0
 // (x + y is -0 only for two -0 operands), and for any other value v + (-0) = v + (+0).
 template <int FMT>
-__device__ __forceinline__ float fw_product(const char* p, float x) {
-    if constexpr (FMT == QR_FMT_F32) return mul_rn(*reinterpret_cast<const float*>(p), x);
+__device__ __forceinline__ typename FwWeight<FMT>::type fw_weight(const char* p) {  // the weight at p (LDS)
+    if constexpr (FMT == QR_FMT_F32) return *reinterpret_cast<const float*>(p);
     else if constexpr (FMT == QR_FMT_BF16)
-        return mul_rn(__uint_as_float(static_cast<uint32_t>(*reinterpret_cast<const uint16_t*>(p)) << 16), x);
-    else return __builtin_fmaf(static_cast<float>(*reinterpret_cast<const _Float16*>(p)), x, 0.0f);
+        return __uint_as_float(static_cast<uint32_t>(*reinterpret_cast<const uint16_t*>(p)) << 16);
+    else return *reinterpret_cast<const _Float16*>(p);
+}
+template <int FMT>
+__device__ __forceinline__ float fw_product(typename FwWeight<FMT>::type w, float x) {
+    if constexpr (FMT == QR_FMT_F16) return __builtin_fmaf(static_cast<float>(w), x, 0.0f);
+    else return mul_rn(w, x);
 }
 
 // Matrices of one launch: workgroups start[m] .. start[m + 1] - 1 take matrix m (a single
@@ -730,9 +995,9 @@ struct FwGroup {
     float* y[kMatVecGroupMax];
 };
 
-template <int FMT, int R>
+template <int FMT, int R, int NV>
 __global__ __launch_bounds__(64) void matvec_fp_wave(MatVecArgs a, FwGroup gr) {
-    using Gm = FwGeom<FMT, R>;
+    using Gm = FwGeom<FMT, R, NV>;
     __shared__ __align__(16) char ring[kFwSlots][Gm::SLOT];
     const int lane = threadIdx.x;
     const int rr = lane >> 3, L = lane & 7;
@@ -744,8 +1009,7 @@ __global__ __launch_bounds__(64) void matvec_fp_wave(MatVecArgs a, FwGroup gr) {
     a.rows = gr.rows[mg];
     a.y = gr.y[mg];
     const long long r0 = static_cast<long long>(static_cast<int>(blockIdx.x) - gr.start[mg]) * R;
-    const int q = blockIdx.y;
-    const float* x = a.x + static_cast<long long>(q) * a.cols;
+    const int q = static_cast<int>(blockIdx.y) * NV;
     const int nch = a.cols / 8;
     const int nseg = (nch + Gm::SEG - 1) / Gm::SEG;
     const int rbytes = nch * Gm::B;
@@ -757,8 +1021,13 @@ __global__ __launch_bounds__(64) void matvec_fp_wave(MatVecArgs a, FwGroup gr) {
         rs[r] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.w + (in ? (r0 + r) * a.row_bytes : 0)),
                                                   static_cast<short>(0), in ? rbytes : 0, kBufferFlags);
     }
-    const __amdgpu_buffer_rsrc_t rsx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), static_cast<short>(0),
-                                                                        nch * 32, kBufferFlags);
+    const float* xs[NV];  // vectors past the last repeat it and are not stored
+    __amdgpu_buffer_rsrc_t rsx[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        xs[v] = a.x + static_cast<long long>(min(q + v, a.nq - 1)) * a.cols;
+        rsx[v] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xs[v]), static_cast<short>(0), nch * 32, kBufferFlags);
+    }
     // segment s into slot s % kFwSlots; past the last segment the last one is read again, so
     // that every round issues the same number of DMAs
     auto issue = [&](int s) {
@@ -770,12 +1039,14 @@ __global__ __launch_bounds__(64) void matvec_fp_wave(MatVecArgs a, FwGroup gr) {
             buffer_load_lds16<kCacheNt>(rs[r], slot + r * kFwRowPad, static_cast<uint32_t>(16 * lane),
                                         static_cast<uint32_t>(s * 1024));
 #pragma unroll
-        for (int i = 0; i < Gm::XDMA; ++i)
-            buffer_load_lds16(rsx, slot + R * kFwRowPad + 1024 * i, static_cast<uint32_t>(16 * lane),
-                              static_cast<uint32_t>(s * Gm::XBYTES + 1024 * i));
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+            for (int i = 0; i < Gm::XDMA; ++i)
+                buffer_load_lds16(rsx[v], slot + R * kFwRowPad + v * Gm::XBYTES + 1024 * i,
+                                  static_cast<uint32_t>(16 * lane), static_cast<uint32_t>(s * Gm::XBYTES + 1024 * i));
     };
 
-    float acc = 0.0f;
+    float acc[NV] = {};
     const int wofs = rr * kFwRowPad + (FMT == QR_FMT_F32 ? 4 : 2) * L;
     const int xofs = R * kFwRowPad + 4 * L;
 #pragma unroll
@@ -787,40 +1058,45 @@ __global__ __launch_bounds__(64) void matvec_fp_wave(MatVecArgs a, FwGroup gr) {
         asm volatile("" ::: "memory");
         const char* slot = ring[s % kFwSlots];
         const int n = min(Gm::SEG, nch - s * Gm::SEG);
+        auto chunk = [&](int c) __attribute__((always_inline)) {
+            const auto w = fw_weight<FMT>(slot + wofs + c * Gm::B);
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                acc[v] = add_rn(acc[v], fw_product<FMT>(w, *reinterpret_cast<const float*>(slot + xofs + v * Gm::XBYTES + c * 32)));
+        };
         if (n == Gm::SEG) {
 #pragma unroll 16
-            for (int c = 0; c < Gm::SEG; ++c)
-                acc = add_rn(acc, fw_product<FMT>(slot + wofs + c * Gm::B,
-                                                  *reinterpret_cast<const float*>(slot + xofs + c * 32)));
+            for (int c = 0; c < Gm::SEG; ++c) chunk(c);
         } else {
-            for (int c = 0; c < n; ++c)
-                acc = add_rn(acc, fw_product<FMT>(slot + wofs + c * Gm::B,
-                                                  *reinterpret_cast<const float*>(slot + xofs + c * 32)));
+            for (int c = 0; c < n; ++c) chunk(c);
         }
         asm volatile("" ::: "memory");  // this slot's reads stay before its refill
     }
     wait_dma();
     // HSum in lane order over the row's 8 lanes
     const int base = lane & ~7;
-    float sum = 0.0f;
-#pragma unroll
-    for (int l = 0; l < 8; ++l) sum = add_rn(sum, __shfl(acc, base + l, 64));
     const long long row = r0 + rr;
-    if constexpr (FMT == QR_FMT_F16) {
-        if (!isfinite(sum) && rr < R && row < a.rows) {
-            // exact decode of the row's lane chain (HalfBitsToFloat, DotKernels.cs:86-100)
-            const uint8_t* w = a.w + row * a.row_bytes;
-            float e = 0.0f;
-            for (int c = 0; c < nch; ++c) {
-                const int k = 8 * c + L;
-                e = add_rn(e, mul_rn(f16_dot_decode(*reinterpret_cast<const uint16_t*>(w + 2 * k)), x[k]));
-            }
-            sum = 0.0f;
 #pragma unroll
-            for (int l = 0; l < 8; ++l) sum = add_rn(sum, __shfl(e, base + l, 64));
+    for (int v = 0; v < NV; ++v) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int l = 0; l < 8; ++l) sum = add_rn(sum, __shfl(acc[v], base + l, 64));
+        if constexpr (FMT == QR_FMT_F16) {
+            if (!isfinite(sum) && rr < R && row < a.rows) {
+                // exact decode of the row's lane chain (HalfBitsToFloat, DotKernels.cs:86-100)
+                const uint8_t* w = a.w + row * a.row_bytes;
+                float e = 0.0f;
+                for (int c = 0; c < nch; ++c) {
+                    const int k = 8 * c + L;
+                    e = add_rn(e, mul_rn(f16_dot_decode(*reinterpret_cast<const uint16_t*>(w + 2 * k)), xs[v][k]));
+                }
+                sum = 0.0f;
+#pragma unroll
+                for (int l = 0; l < 8; ++l) sum = add_rn(sum, __shfl(e, base + l, 64));
+            }
         }
+        if (L == 0 && rr < R && row < a.rows && q + v < a.nq) a.y[static_cast<long long>(q + v) * a.rows + row] = sum;
     }
-    if (L == 0 && rr < R && row < a.rows) a.y[static_cast<long long>(q) * a.rows + row] = sum;
 }
 
 // fp weight k of a staged row
@@ -1288,6 +1564,85 @@ bool blk_ring_launch(const MatVecArgs* a, int n, hipStream_t stream, hipError_t*
     return true;
 }
 
+// Several vectors of the block formats (matvec_blk_multi), for one matrix or a group that
+// shares x: false when the shape does not fit it (up to 512 items a row, whole item pairs, rows
+// and x aligned as the policies read them, the terms of a workgroup's tiles in LDS).
+template <class Pol, int NV>
+hipError_t multi_launch_nv(const MatVecArgs& a, const MvMulti& k, const BlkGroup& gr, int threads, size_t lds,
+                           hipStream_t stream) {
+    static bool attr = false;  // dynamic LDS above 64 KiB must be allowed per kernel
+    if (lds > 64 * 1024 && !attr) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&matvec_blk_multi<Pol, NV>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return e;
+        attr = true;
+    }
+    const dim3 grid(static_cast<unsigned>((gr.start[gr.n] + 7) / 8 * 8 * k.passes));
+    hipLaunchKernelGGL((matvec_blk_multi<Pol, NV>), grid, dim3(threads), lds, stream, a, k, gr);
+    return hipGetLastError();
+}
+
+template <class Pol>
+bool blk_multi_launch_pol(const MatVecArgs* a, int n, hipStream_t stream, hipError_t* err) {
+    const int align = Pol::kAlign;
+    for (int m = 0; m < n; ++m)
+        if (reinterpret_cast<uintptr_t>(a[m].x) % 16 || a[m].cols % 64 ||
+            reinterpret_cast<uintptr_t>(a[m].w) % align || a[m].row_bytes % align || a[m].rows < 1)
+            return false;
+    MvMulti k{};
+    k.P = a[0].cols / 32;
+    if (k.P > 512) return false;
+    k.tpg = (k.P + 31) / 32 * 32;
+    k.R = std::max(1, kMvThreads / k.tpg);
+    const int threads = (k.R * k.tpg + 63) / 64 * 64;
+    k.tstride = (k.P + 3) / 4 * 4 + 4;
+    k.slot_bytes = threads / 64 * kMulUnits<Pol> * 1024;
+    for (int m = 0; m < n; ++m)
+        if (a[m].rows >= (1LL << 31) - k.R) return false;
+    // vectors spread evenly over the fewest passes of at most four
+    k.passes = (a[0].nq + 3) / 4;
+    const int nv = (a[0].nq + k.passes - 1) / k.passes;
+    BlkGroup gr = group_of(a, n, k.R);
+    // Every workgroup is resident at once (each loads its x once and walks many tiles): eight
+    // waves per CU, which the registers of four vectors allow, and on each XCD whole sets of
+    // passes -- one workgroup more than fits would run a second round (w_down of 14336 columns,
+    // 7 waves a workgroup: 105 us with 1.2 workgroups per CU, 59 with one).
+    const int per_cu = std::max(1, 512 / threads);
+    group_grid(gr, 8 * std::max(1, 32 * per_cu / k.passes), 0, 0, 1);
+    int most = 1;  // tiles of a workgroup
+    for (int m = 0; m < n; ++m) {
+        const int G = gr.start[m + 1] - gr.start[m];
+        most = std::max(most, (gr.ntiles[m] + G - 1) / G);
+    }
+    const int ring = kMulSlots * k.slot_bytes, per_tile = k.R * nv * k.tstride * 4;
+    k.flush = std::min(most, std::max(1, (160 * 1024 / per_cu - ring) / per_tile));
+    const size_t lds = static_cast<size_t>(ring) + static_cast<size_t>(k.flush) * per_tile;
+    if (lds > 160 * 1024) return false;
+    if constexpr (std::is_same<Pol, MulQ40>::value) {
+        if (nv == 1) {
+            *err = multi_launch_nv<Pol, 1>(a[0], k, gr, threads, lds, stream);
+            return true;
+        }
+    }
+    switch (nv) {
+    case 2: *err = multi_launch_nv<Pol, 2>(a[0], k, gr, threads, lds, stream); break;
+    case 3: *err = multi_launch_nv<Pol, 3>(a[0], k, gr, threads, lds, stream); break;
+    default: *err = multi_launch_nv<Pol, 4>(a[0], k, gr, threads, lds, stream); break;
+    }
+    return true;
+}
+
+bool blk_multi_launch(const MatVecArgs* a, int n, hipStream_t stream, hipError_t* err) {
+    // a single vector of Q8_0 and Q4_K has its own forms
+    if (a[0].nq < 2 && a[0].fmt != QR_FMT_Q4_0) return false;
+    switch (a[0].fmt) {
+    case QR_FMT_Q8_0: return blk_multi_launch_pol<MulQ8>(a, n, stream, err);
+    case QR_FMT_Q4_0: return blk_multi_launch_pol<MulQ40>(a, n, stream, err);
+    case QR_FMT_Q4_K: return blk_multi_launch_pol<MulQ4K>(a, n, stream, err);
+    default: return false;
+    }
+}
+
 // The persistent form for Q4_K (64-column items: rows of at most 512 items, 32768 columns) and
 // Q8_0 (block pairs: whole pairs and 4-byte aligned rows): false when the shape does not fit or
 // the terms of a workgroup's tiles would not fit in 64 KiB of LDS.
@@ -1385,8 +1740,19 @@ bool fp_wave_fits(const MatVecArgs& a) {
 
 template <int FMT>
 hipError_t launch_fp_group(const MatVecArgs& a, const FwGroup& g, hipStream_t stream) {
-    const dim3 grid(static_cast<unsigned>(g.start[g.n]), static_cast<unsigned>(a.nq));
-    hipLaunchKernelGGL((matvec_fp_wave<FMT, 8>), grid, dim3(64), 0, stream, a, g);
+    // Vectors per wave: as few as keep every wave resident at once (six one-wave workgroups per
+    // CU at two vectors), up to four, spread evenly.  Sharing saves reads of the weights but
+    // makes each wave's serial walk longer: 2048-column F16 layers whose waves all fit (4
+    // vectors) took 61.4 us unshared and 66.7 at four per wave; 5632 rows x 30 vectors of BF16
+    // 343 unshared and 232 shared.
+    const int fit = static_cast<int>(std::max(1LL, 1536LL / std::max(1, g.start[g.n])));
+    const int least = std::min(4, (a.nq + fit - 1) / fit);
+    const int passes = (a.nq + least - 1) / least, nv = (a.nq + passes - 1) / passes;
+    const dim3 grid(static_cast<unsigned>(g.start[g.n]), static_cast<unsigned>(passes));
+    if (nv == 1) hipLaunchKernelGGL((matvec_fp_wave<FMT, 8, 1>), grid, dim3(64), 0, stream, a, g);
+    else if (nv == 2) hipLaunchKernelGGL((matvec_fp_wave<FMT, 8, 2>), grid, dim3(64), 0, stream, a, g);
+    else if (nv == 3) hipLaunchKernelGGL((matvec_fp_wave<FMT, 8, 3>), grid, dim3(64), 0, stream, a, g);
+    else hipLaunchKernelGGL((matvec_fp_wave<FMT, 8, 4>), grid, dim3(64), 0, stream, a, g);
     return hipGetLastError();
 }
 
@@ -1404,6 +1770,8 @@ hipError_t launch_fp(const MatVecArgs& a, hipStream_t stream) {
 
 hipError_t launch_matvec(const MatVecArgs& a, hipStream_t stream) {
     if (a.nq == 0 || a.rows == 0) return hipSuccess;
+    hipError_t multi;
+    if (blk_multi_launch(&a, 1, stream, &multi)) return multi;
     switch (a.fmt) {
     case QR_FMT_F32: return launch_fp<QR_FMT_F32>(a, stream);
     case QR_FMT_F16: return launch_fp<QR_FMT_F16>(a, stream);
@@ -1441,6 +1809,7 @@ hipError_t launch_matvec_group(const MatVecArgs* a, int n, hipStream_t stream) {
             same = same && a[m].fmt == a[0].fmt && a[m].cols == a[0].cols && a[m].row_bytes == a[0].row_bytes &&
                    a[m].x == a[0].x && a[m].nq == a[0].nq;
         hipError_t e = hipSuccess;
+        if (same && blk_multi_launch(a, n, stream, &e)) return e;
         if (same && a[0].fmt == QR_FMT_Q8_0 && (blk_ring_launch(a, n, stream, &e) || blk_persistent_launch(a, n, stream, &e)))
             return e;
         if (same && a[0].fmt == QR_FMT_Q4_K && blk_persistent_launch(a, n, stream, &e)) return e;

@@ -22,7 +22,8 @@ struct MatVecArgs {
 bool matvec_shape_ok(int fmt, int cols);
 hipError_t launch_matvec(const MatVecArgs& a, hipStream_t stream);
 // n <= kMatVecGroupMax MatVecs that read the same x (same format, cols and nq): one launch
-// when the format streams rows in the single-wave form (F32/F16/BF16), else one per matrix;
+// when a kernel takes the shape as a group (all but Q6_K and rows of odd items), else one per
+// matrix;
 // every y equals launch_matvec's.
 constexpr int kMatVecGroupMax = 4;
 hipError_t launch_matvec_group(const MatVecArgs* a, int n, hipStream_t stream);

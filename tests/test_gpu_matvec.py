@@ -100,6 +100,39 @@ def test_matvec_long_rows_and_many_tiles(gpu, fmt, rows, cols, nq):
     assert_exact(got, want, f"{fmt} {rows}x{cols} nq{nq}")
 
 
+@pytest.mark.parametrize("nq", [2, 3, 5, 8, 9])
+@pytest.mark.parametrize("fmt,rows,cols", [
+    ("Q8_0", 37, 64), ("Q8_0", 300, 4096), ("Q8_0", 5, 16384), ("Q8_0", 3, 16448),  # 1, 64 and 256 pairs; one past
+    ("Q4_0", 130, 192), ("Q4_0", 41, 2816), ("Q4_0", 9, 1056),                      # 88 items; odd items: not this form
+    ("Q4_K", 37, 256), ("Q4_K", 2100, 1024), ("Q4_K", 6, 14336),
+    ("F16", 21, 2048), ("BF16", 9, 520), ("F32", 17, 1032), ("Q6_K", 11, 1024),
+])
+def test_matvec_several_vectors(gpu, fmt, rows, cols, nq):
+    """Vectors that share one pass over the weights: even and ragged groups of up to four, rows
+    that do not fill a tile, the fewest and most items of a row."""
+    got, want, _, _ = run(fmt, rows, cols, nq, seed=rows + cols + nq)
+    assert_exact(got, want, f"{fmt} {rows}x{cols} nq{nq}")
+
+
+@pytest.mark.parametrize("fmt", ["Q8_0", "Q4_0", "Q4_K", "F16", "BF16", "F32"])
+def test_matvec_several_vectors_extremes(gpu, fmt):
+    """Infinities, NaN, zeros of both signs and huge values in x, and weights of random bytes:
+    each vector of four equals the same vector alone."""
+    code, rows, cols = quant.FMT[fmt], 70, 512
+    raw = np.random.default_rng(8).integers(0, 256, rows * quant.random_rows(code, 1, cols, 1, 0.05)[0].size, dtype=np.uint8)
+    x = normal(9, (4, cols))
+    x[1, ::3] = -0.0
+    x[2, 5], x[2, 77] = np.inf, np.nan
+    x[3] *= np.float32(1e30)
+    w, xd = dev(raw), dev(x)
+    y = torch.empty((4, rows), device="cuda")
+    qr.matvec_dev(w, code, rows, cols, xd, y)
+    for v in range(4):
+        one = torch.empty((1, rows), device="cuda")
+        qr.matvec_dev(w, code, rows, cols, xd[v:v + 1].contiguous(), one)
+        assert_exact_nan(y[v].cpu().numpy(), one[0].cpu().numpy(), f"{fmt} vector {v}")
+
+
 def assert_exact_nan(got, want, what):
     """Bit-exact, except that any NaN matches any NaN (payloads are not compared)."""
     g, w = got.reshape(-1), want.reshape(-1)
