@@ -6,6 +6,8 @@
 // head_dim run per kv head, converted to the cache dtype on the way.
 #include "qr_kernels.hpp"
 
+#include <algorithm>
+
 namespace qr {
 namespace {
 
@@ -255,6 +257,105 @@ __global__ void __launch_bounds__(kRopeThreads) rope_append_items_kernel(const R
     }
 }
 
+// One thread: the pages that a device-side position needs, from the pool's device counter.
+// Returns the pool page of the last of the a.n positions, -1 where it could not be had.
+__device__ __forceinline__ int claim_pages(const PageClaimArgs& a) {
+    const int pos = *a.pos_dev;
+    if (pos < 0 || pos > a.max_seq - a.n) {
+        atomicOr(&a.state[1], 2);
+        return -1;
+    }
+    const int need = ((pos + a.n - 1) >> kPageShift) + 1;
+    const int held = a.state[a.held_index];
+    int page = a.page_table[need - 1];  // read along with held: valid only if the page is held
+    if (need > held) {
+        const int cnt = need - held;
+        const int first = atomicAdd(&a.state[0], cnt);
+        if (first + cnt > a.capacity) {
+            atomicSub(&a.state[0], cnt);
+            atomicOr(&a.state[1], 1);
+            return -1;
+        }
+        for (int i = 0; i < cnt; ++i) a.page_table[held + i] = first + i;
+        a.state[a.held_index] = need;
+        page = first + cnt - 1;
+    }
+    atomicMax(&a.state[a.seq_index], pos + a.n);  // PagedKvCache.cs:68
+    return page;
+}
+
+// One position at a device-side index: page claim, RoPE and append in one workgroup.  The item
+// kernel needs the claim of a launch before it, two launches of one workgroup each (plus V
+// tiles) whose time is their latency: in a captured step of the 8B shape (fp16, 32 + 8 heads of
+// 128) 3.5 and 6.5 us per layer.  Here thread 0 claims while the others read their rows and the
+// cos/sin of the position are computed: QQ us.  Items are 8 dims (d .. d + 3 and d + D/2 ..
+// d + D/2 + 3) of a K, q or V head, the arithmetic that of the item kernel.
+constexpr int kRopeStepThreads = 1024;
+template <int IPT>
+__global__ void __launch_bounds__(kRopeStepThreads) rope_step_kernel(const RopeAppendArgs a, const PageClaimArgs c) {
+    const AppendArgs& g = a.app;
+    __shared__ float cs[2 * kMaxRopeHalf];  // cos, then sin
+    __shared__ int page;
+    const int D = g.geom.head_dim;
+    const int half = D >> 1;
+    const int kv_heads = g.geom.kv_heads;
+    const int rot_heads = kv_heads + (a.q ? a.q_width / D : 0);  // K, then q
+    const int per_head = half / 4;
+    const int nitems = (rot_heads + kv_heads) * per_head;        // and V
+    const int pos = *g.pos_dev;
+    float4 x0[IPT], x1[IPT];
+    auto source = [&](int h) -> float* {
+        if (h < kv_heads) return const_cast<float*>(static_cast<const float*>(g.src[0])) + h * D;
+        if (h < rot_heads) return a.q + (h - kv_heads) * D;
+        return const_cast<float*>(static_cast<const float*>(g.src[1])) + (h - rot_heads) * D;
+    };
+#pragma unroll
+    for (int k = 0; k < IPT; ++k) {
+        const int it = min(static_cast<int>(threadIdx.x + blockDim.x * k), nitems - 1);  // past the end: a valid item, not stored
+        const int h = it / per_head;
+        const float* src = source(h) + 4 * (it - h * per_head);
+        x0[k] = *reinterpret_cast<const float4*>(src);
+        x1[k] = *reinterpret_cast<const float4*>(src + half);
+    }
+    // the last wave's first thread claims; the cos/sin go to the first threads
+    if (threadIdx.x == blockDim.x - 64) page = claim_pages(c);
+    for (int i = threadIdx.x; i < D; i += blockDim.x) {
+        const float ang = mul_rn(static_cast<float>(pos), a.freq[i < half ? i : i - half]);
+        cs[i] = i < half ? cosf(ang) : sinf(ang);
+    }
+    __syncthreads();
+    if (page < 0) return;  // nothing is written, q keeps its values
+    const int slot = pos & (kPageTokens - 1);
+#pragma unroll
+    for (int k = 0; k < IPT; ++k) {
+        const int it = threadIdx.x + blockDim.x * k;
+        if (it >= nitems) break;
+        const int h = it / per_head;
+        const int d = 4 * (it - h * per_head);
+        const float a0[4] = {x0[k].x, x0[k].y, x0[k].z, x0[k].w}, a1[4] = {x1[k].x, x1[k].y, x1[k].z, x1[k].w};
+        if (h >= rot_heads) {
+            store4(g.pool, g.dtype, g.geom, page, 1, h - rot_heads, slot, d, a0);
+            store4(g.pool, g.dtype, g.geom, page, 1, h - rot_heads, slot, d + half, a1);
+            continue;
+        }
+        float y0[4], y1[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float cc = cs[d + e], ss = cs[half + d + e];
+            y0[e] = sub_rn(mul_rn(a0[e], cc), mul_rn(a1[e], ss));
+            y1[e] = add_rn(mul_rn(a0[e], ss), mul_rn(a1[e], cc));
+        }
+        if (h < kv_heads) {
+            store4(g.pool, g.dtype, g.geom, page, 0, h, slot, d, y0);
+            store4(g.pool, g.dtype, g.geom, page, 0, h, slot, d + half, y1);
+        } else {
+            float* q = source(h);
+            *reinterpret_cast<float4*>(q + d) = make_float4(y0[0], y0[1], y0[2], y0[3]);
+            *reinterpret_cast<float4*>(q + d + half) = make_float4(y1[0], y1[1], y1[2], y1[3]);
+        }
+    }
+}
+
 __global__ void __launch_bounds__(256) rope_append_kernel(const RopeAppendArgs a) {
     const AppendArgs& g = a.app;
     const int D = g.geom.head_dim;
@@ -398,28 +499,8 @@ hipError_t launch_append(const AppendArgs& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// One thread: the pages a device-side position needs, from the pool's device counter.
 __global__ void __launch_bounds__(64) page_claim_kernel(const PageClaimArgs a) {
-    if (threadIdx.x != 0) return;
-    const int pos = *a.pos_dev;
-    if (pos < 0 || pos > a.max_seq - a.n) {
-        atomicOr(&a.state[1], 2);
-        return;
-    }
-    const int need = ((pos + a.n - 1) >> kPageShift) + 1;
-    const int held = a.state[a.held_index];
-    if (need > held) {
-        const int cnt = need - held;
-        const int first = atomicAdd(&a.state[0], cnt);
-        if (first + cnt > a.capacity) {
-            atomicSub(&a.state[0], cnt);
-            atomicOr(&a.state[1], 1);
-            return;
-        }
-        for (int i = 0; i < cnt; ++i) a.page_table[held + i] = first + i;
-        a.state[a.held_index] = need;
-    }
-    atomicMax(&a.state[a.seq_index], pos + a.n);  // PagedKvCache.cs:68
+    if (threadIdx.x == 0) claim_pages(a);
 }
 
 hipError_t launch_page_claim(const PageClaimArgs& a, hipStream_t stream) {
@@ -473,6 +554,22 @@ hipError_t launch_rope_append(const RopeAppendArgs& a, hipStream_t stream) {
         hipLaunchKernelGGL(rope_append_kernel, dim3((a.app.n + kRopeRows - 1) / kRopeRows), dim3(256), 0, stream, a);
     }
 #undef QR_ROPE_ITEMS
+    return hipGetLastError();
+}
+
+hipError_t launch_rope_step(const RopeAppendArgs& a, const PageClaimArgs& c, hipStream_t stream) {
+    const int D = a.app.geom.head_dim;
+    if (a.app.n != 1 || rope_generic(D)) {  // several positions or a generic head size: claim, then append
+        const hipError_t e = launch_page_claim(c, stream);
+        return e != hipSuccess ? e : launch_rope_append(a, stream);
+    }
+    const int heads = a.app.geom.kv_heads + (a.q ? a.q_width / D : 0);
+    if (rope_items_per_thread(heads, D) > kRopeMaxItems) return hipErrorInvalidValue;
+    const int items = (heads + a.app.geom.kv_heads) * (D / 8);  // at most 4 a thread
+    const dim3 block(std::min(kRopeStepThreads, (items + 63) / 64 * 64));
+    if (items <= kRopeStepThreads) hipLaunchKernelGGL((rope_step_kernel<1>), dim3(1), block, 0, stream, a, c);
+    else if (items <= 2 * kRopeStepThreads) hipLaunchKernelGGL((rope_step_kernel<2>), dim3(1), block, 0, stream, a, c);
+    else hipLaunchKernelGGL((rope_step_kernel<4>), dim3(1), block, 0, stream, a, c);
     return hipGetLastError();
 }
 

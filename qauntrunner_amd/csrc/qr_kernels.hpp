@@ -125,6 +125,9 @@ struct RopeAppendArgs {
     float freq[kMaxRopeHalf];
 };
 hipError_t launch_rope_append(const RopeAppendArgs& a, hipStream_t stream);
+// The pages of the rows at the device position a.app.pos_dev (= c.pos_dev), then their RoPE
+// append: one launch for a single position, two otherwise.
+hipError_t launch_rope_step(const RopeAppendArgs& a, const PageClaimArgs& c, hipStream_t stream);
 // One workgroup of kRopeThreads threads per position, each thread taking up to
 // kRopeMaxItems items of 8 dims (K heads plus q heads); wider rows use a row kernel that
 // cannot read the position on the device, so device-position RoPE appends need

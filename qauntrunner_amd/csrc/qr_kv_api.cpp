@@ -727,7 +727,6 @@ int rope_step_dev(qr_kv* kv, int seq_id, int layer, int n, const int* pos_dev, f
     c.max_seq = kv->max_seq;
     c.pos_dev = pos_dev;
     c.n = n;
-    QR_HIP(launch_page_claim(c, st));
     RopeAppendArgs a{};
     a.app.pool = kv->store.pool();
     a.app.page_table = kv->store.page_table_dev() + kv->store.pt_offset(seq_id, layer);
@@ -748,7 +747,7 @@ int rope_step_dev(qr_kv* kv, int seq_id, int layer, int n, const int* pos_dev, f
     a.q_width = kv->heads * kv->head_dim;
     const int half = kv->head_dim / 2;
     for (int i = 0; i < half; ++i) a.freq[i] = std::pow(theta, (-2.0f * static_cast<float>(i)) / static_cast<float>(kv->head_dim));
-    QR_HIP(launch_rope_append(a, st));
+    QR_HIP(launch_rope_step(a, c, st));
     kv->store.mark_device_ahead();
     if (cap) kv->store.mark_replayable();
     return QR_OK;

@@ -548,3 +548,35 @@ def test_no_alloc_decode_is_captured_after_a_device_step(gpu):
             torch.cuda.synchronize()
             assert torch.equal(out, want)
         assert kv.SeqLen == p0 + 1
+
+
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,with_q", [
+    ("f32", 1, 1, 8, True),        # three items: most of the one wave idle
+    ("bf16", 8, 2, 64, False),     # K and V only
+    ("f16", 32, 16, 128, True),    # exactly 1024 items: one a thread
+    ("f16", 24, 8, 256, True),     # 1280 items: two a thread
+    ("f32", 48, 16, 256, True),    # 2560 items: four a thread, the widest row
+    ("bf16", 28, 4, 96, True),
+])
+def test_rope_step_writes_what_the_host_path_writes(gpu, dtype, heads, kv_heads, D, with_q):
+    """The one-launch claim + RoPE + append, across a page boundary: rows and rotated q equal to
+    AppendRopeDev's, bit for bit."""
+    import torch
+
+    n, p0 = 4, 254
+    Q, K, V = _rows(D + heads, p0 + n, heads, kv_heads, D)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    with qr.PagedKvCache(1, heads, kv_heads, D, 1000, kv_dtype=dtype) as A, \
+            qr.PagedKvCache(1, heads, kv_heads, D, 1000, kv_dtype=dtype) as B:
+        for kv in (A, B):
+            kv.AppendRopeDev(0, 0, dev(Q[:p0]), dev(K[:p0]), dev(V[:p0]), THETA)
+        pos = torch.zeros(1, dtype=torch.int32, device=gpu)
+        for t in range(p0, p0 + n):
+            qa, qb = (dev(Q[t]), dev(Q[t])) if with_q else (None, None)
+            A.AppendRopeDev(0, t, qa, dev(K[t]), dev(V[t]), THETA)
+            pos.fill_(t)
+            B.AppendRopeStepDev(0, pos, qb, dev(K[t]), dev(V[t]), THETA)
+            assert not with_q or torch.equal(qa, qb)
+        assert A.SeqLen == B.SeqLen == p0 + n and A.BytesUsed == B.BytesUsed
+        for a, b in zip(A.Read(0, 0, p0 + n), B.Read(0, 0, p0 + n)):
+            assert np.array_equal(a, b)
