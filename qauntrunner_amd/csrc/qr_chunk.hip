@@ -23,7 +23,7 @@
 // PV k-slots of step ks.
 // Operands stay in the cache's 16-bit type (no conversion); q enters as hi + lo parts
 // when its own type is not the cache's (fp32 queries keep ~22 or ~16 bits), P is
-// rounded to the cache type; accumulation and softmax are fp32.  Row sums come from
+// rounded to the cache type (groups that are not a power of two: hi + lo parts); accumulation and softmax are fp32.  Row sums come from
 // the MFMA too (a ones operand), consistent with the rounded P of the numerator.
 // The causal mask is applied only on tiles that reach past the block's first query.
 #include "qr_chunk.hpp"
@@ -35,9 +35,7 @@ namespace qr {
 namespace {
 
 constexpr int kTile = 64;  // positions per tile
-#ifndef QR_CHUNK_MAX_NT
-#define QR_CHUNK_MAX_NT 2
-#endif
+constexpr int kMaxNT = 2;  // 16-row N tiles per wave (four measured slower)
 
 // Elements 32kk + 8q4 + i (kk < NK, i < 8) of the q row starting at element `row`, as fp32.
 // The dtype branch sits outside the loads, so all of them are issued before the first is
@@ -74,7 +72,6 @@ struct ChunkK {
     int kv_heads;
     int heads;
     int group;
-    int group_shift;         // log2(group)
     int pos0;
     const int* pos0_dev;     // device position of query 0 (clamped to [0, pos0]) when set
     int nq;
@@ -134,9 +131,11 @@ __device__ __forceinline__ float max_quarters(float x) {
 
 // BF16: cache element type; NT: 16-row N tiles per wave; NSTAGE: LDS tile buffers;
 // QSPLIT: q is not exact in the cache type and enters as hi + lo parts.
-template <bool BF16, int D, int NT, int NSTAGE, bool QSPLIT>
+// PSPLIT: P enters PV as hi + lo parts too (and the row sums are of both), as in the decode
+// kernel that served the shape before.
+template <bool BF16, int D, int NT, int NSTAGE, bool QSPLIT, bool PSPLIT>
 // Workgroups per CU: two at NT <= 2 with two LDS stages (64 KiB); one with three stages
-// (96 KiB of LDS) or NT = 4 (registers).  NT = 1 runs eight waves per workgroup.
+// (96 KiB of LDS).  NT = 1 runs eight waves per workgroup.
 __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 2 : 1) chunk_tile_kernel(const ChunkK p) {
     using T = typename std::conditional<BF16, __bf16, _Float16>::type;
     typedef T vec8 __attribute__((ext_vector_type(8)));
@@ -182,16 +181,17 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
     const int q4 = lane >> 4;
     const int col = lane & 15;
 
-    // rows of this lane, one per N tile: (query, head) = (rho >> log2 G, rho & (G - 1))
+    // rows of this lane, one per N tile: (query, head) = (rho / G, rho % G)
     const int q_first = qblk * p.queries_per_block;
     int row_q[NT], row_h[NT];
     bool row_on[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         const int rho = rw * 16 * NT + j * 16 + col;
-        row_q[j] = q_first + (rho >> p.group_shift);
-        row_h[j] = kvh * p.group + (rho & (p.group - 1));
-        row_on[j] = row_q[j] < p.nq && (rho >> p.group_shift) < p.queries_per_block;
+        const int dq = rho / p.group;
+        row_q[j] = q_first + dq;
+        row_h[j] = kvh * p.group + (rho - dq * p.group);
+        row_on[j] = row_q[j] < p.nq && dq < p.queries_per_block;
     }
     const int q_last = min(p.nq, q_first + p.queries_per_block) - 1;
     const int pos0 = chunk_pos0(p);
@@ -405,7 +405,7 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
                 for (int t = 0; t < NDT; ++t) acc[j][t] *= corr;
             }
         }
-        vec8 pb[NT][NKS];
+        vec8 pb[NT][NKS], pl[NT][NKS];
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             if (grow[j]) m[j] = ts[j];
@@ -413,8 +413,12 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
 #pragma unroll
             for (int lm = 0; lm < NMT; ++lm)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    pb[j][lm >> 1][4 * (lm & 1) + r] = static_cast<T>(fast_exp2(fmaf(sc[j][lm][r], sscale[j], mneg)));
+                for (int r = 0; r < 4; ++r) {
+                    const float e = fast_exp2(fmaf(sc[j][lm][r], sscale[j], mneg));
+                    const T hi = static_cast<T>(e);
+                    pb[j][lm >> 1][4 * (lm & 1) + r] = hi;
+                    if (PSPLIT) pl[j][lm >> 1][4 * (lm & 1) + r] = static_cast<T>(e - static_cast<float>(hi));
+                }
         }
 
         // ---- PV (and the row sums: a ones operand turns the MFMA into sum over positions).
@@ -429,11 +433,17 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
                 va[dt] = *reinterpret_cast<const vec8*>(vt + SB * ks + 1024 * dt + 16 * lane);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < NT; ++j) accl[j] = mfma16(ones, pb[j][kq], accl[j]);
+            for (int j = 0; j < NT; ++j) {
+                accl[j] = mfma16(ones, pb[j][kq], accl[j]);
+                if (PSPLIT) accl[j] = mfma16(ones, pl[j][kq], accl[j]);
+            }
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-                for (int j = 0; j < NT; ++j) acc[j][dt] = mfma16(va[dt], pb[j][kq], acc[j][dt]);
+                for (int j = 0; j < NT; ++j) {
+                    acc[j][dt] = mfma16(va[dt], pb[j][kq], acc[j][dt]);
+                    if (PSPLIT) acc[j][dt] = mfma16(va[dt], pl[j][kq], acc[j][dt]);
+                }
         }
     }
 
@@ -528,29 +538,21 @@ int cu_total() {
     return n;
 }
 
-template <bool BF, int D, int NT, int NSTAGE>
+template <bool BF, int D, int NT, int NSTAGE, bool PSPLIT>
 hipError_t launch_q(const ChunkK& k, bool qsplit, dim3 grid, hipStream_t s) {
-    if constexpr (NT == 4 && D == 128) {  // hi + lo queries there would spill: the plan never asks
-        if (qsplit) return hipErrorInvalidValue;
-    } else {
-        if (qsplit) {
-            hipLaunchKernelGGL((chunk_tile_kernel<BF, D, NT, NSTAGE, true>), grid, dim3(NT == 1 ? 512 : 256), 0, s, k);
-            return hipGetLastError();
-        }
-    }
-    hipLaunchKernelGGL((chunk_tile_kernel<BF, D, NT, NSTAGE, false>), grid, dim3(NT == 1 ? 512 : 256), 0, s, k);
+    const dim3 block(NT == 1 ? 512 : 256);
+    if (qsplit) hipLaunchKernelGGL((chunk_tile_kernel<BF, D, NT, NSTAGE, true, PSPLIT>), grid, block, 0, s, k);
+    else hipLaunchKernelGGL((chunk_tile_kernel<BF, D, NT, NSTAGE, false, PSPLIT>), grid, block, 0, s, k);
     return hipGetLastError();
 }
 
-// NT 4 and 2 (prefill-sized query blocks) are MFMA-bound and double buffer; NT 1 (a
-// few queries, e.g. speculative verify) streams the cache and keeps three tiles in LDS.
+// NT 2 (prefill-sized query blocks) is MFMA-bound and double buffers; NT 1 (a few queries,
+// e.g. speculative verify) streams the cache and keeps three tiles in LDS.
 template <bool BF, int D>
-hipError_t launch_nt(const ChunkK& k, int nt, bool qsplit, dim3 grid, hipStream_t s) {
-    switch (nt) {
-        case 1: return launch_q<BF, D, 1, 3>(k, qsplit, grid, s);
-        case 2: return launch_q<BF, D, 2, 2>(k, qsplit, grid, s);
-        default: return launch_q<BF, D, 4, 2>(k, qsplit, grid, s);
-    }
+hipError_t launch_nt(const ChunkK& k, int nt, bool qsplit, bool psplit, dim3 grid, hipStream_t s) {
+    if (nt == 1)
+        return psplit ? launch_q<BF, D, 1, 3, true>(k, qsplit, grid, s) : launch_q<BF, D, 1, 3, false>(k, qsplit, grid, s);
+    return psplit ? launch_q<BF, D, 2, 2, true>(k, qsplit, grid, s) : launch_q<BF, D, 2, 2, false>(k, qsplit, grid, s);
 }
 
 }  // namespace
@@ -561,13 +563,28 @@ bool chunk_mfma_eligible(int kv_dtype, int head_dim, int heads, int kv_heads) {
     return g <= 64 && (g & (g - 1)) == 0;
 }
 
+// Groups that are not a power of two (24 heads over 8, 28 over 4): P in hi + lo parts.  They ran
+// as one decode entry per query, every query reading its own K/V: 500 queries after 1000
+// positions (28 heads over 4, bf16) took 137 us with the append, here 51, with errors against
+// 64 bits of 4.3e-6 and 2.2e-6.  Few queries over few keys keep the decode entries, which one or
+// two launches of 64 serve, merged in the kernel.  By the K/V bytes that the entries would read
+// themselves: 64 queries at 135 MB 15.9 us as entries against 20.1 here (head_dim 64) and 23.4
+// against 20.4 (head_dim 128), 16 queries at 197 MB 26.3 against 19.1; 128 queries from scratch
+// 17.7 against 19.4, 500 69 against 34.
+bool chunk_mfma_split_eligible(int kv_dtype, int head_dim, int heads, int kv_heads, int pos0, int nq) {
+    if (kv_dtype == QR_DTYPE_F32 || (head_dim != 64 && head_dim != 128) || heads % kv_heads) return false;
+    const int g = heads / kv_heads;
+    if (g > 64 || (g & (g - 1)) == 0) return false;
+    const double bytes = 4.0 * nq * (pos0 + 0.5 * nq) * kv_heads * head_dim;
+    return nq > 128 || (nq > 1 && bytes >= 160e6);
+}
+
 ChunkPlan plan_chunk(const ChunkArgs& a) {
     ChunkPlan pl{};
     const int g = a.heads / a.geom.kv_heads;
     const int total = a.pos0 + a.nq;  // tokens attended by the last query
-    // rows per workgroup: up to 256 (4 queries' worth of heads per wave and N tile)
-    // (hi + lo queries at head_dim 128 need the registers of two N tiles)
-    int nt = QR_CHUNK_MAX_NT;
+    // rows per workgroup: 64 per N tile
+    int nt = kMaxNT;
     while (nt > 1 && (64 * nt) / g > std::max(1, a.nq)) nt >>= 1;
     pl.nt = nt;
     pl.queries_per_block = std::max(1, 64 * nt / g);
@@ -597,9 +614,7 @@ hipError_t launch_chunk(const ChunkArgs& a, const ChunkPlan& pl, void* workspace
     k.kv_heads = a.geom.kv_heads;
     k.heads = a.heads;
     k.group = a.heads / a.geom.kv_heads;
-    int gs = 0;
-    while ((1 << gs) < k.group) ++gs;
-    k.group_shift = gs;
+    const bool psplit = (k.group & (k.group - 1)) != 0;
     k.pos0 = a.pos0;
     k.pos0_dev = a.pos0_dev;
     k.nq = a.nq;
@@ -626,9 +641,9 @@ hipError_t launch_chunk(const ChunkArgs& a, const ChunkPlan& pl, void* workspace
     const bool qsplit = a.q_dtype != a.kv_dtype;  // q not exact in the cache's 16-bit type
     hipError_t e;
     if (a.geom.head_dim == 128)
-        e = bf ? launch_nt<true, 128>(k, pl.nt, qsplit, grid, stream) : launch_nt<false, 128>(k, pl.nt, qsplit, grid, stream);
+        e = bf ? launch_nt<true, 128>(k, pl.nt, qsplit, psplit, grid, stream) : launch_nt<false, 128>(k, pl.nt, qsplit, psplit, grid, stream);
     else
-        e = bf ? launch_nt<true, 64>(k, pl.nt, qsplit, grid, stream) : launch_nt<false, 64>(k, pl.nt, qsplit, grid, stream);
+        e = bf ? launch_nt<true, 64>(k, pl.nt, qsplit, psplit, grid, stream) : launch_nt<false, 64>(k, pl.nt, qsplit, psplit, grid, stream);
     if (e != hipSuccess) return e;
     if (after_split && (e = hipEventRecord(after_split, stream)) != hipSuccess) return e;
     if (pl.splits == 1) return hipSuccess;

@@ -34,6 +34,8 @@ struct ChunkPlan {
 
 // 16-bit cache, head_dim 64 or 128, power-of-two group heads/kv_heads <= 64.
 bool chunk_mfma_eligible(int kv_dtype, int head_dim, int heads, int kv_heads);
+// The same with any other group of up to 64, host positions only.
+bool chunk_mfma_split_eligible(int kv_dtype, int head_dim, int heads, int kv_heads, int pos0, int nq);
 ChunkPlan plan_chunk(const ChunkArgs& a);
 // after_split: when not null, recorded on `stream` right after the main kernel.
 hipError_t launch_chunk(const ChunkArgs& a, const ChunkPlan& plan, void* workspace, hipStream_t stream,

@@ -511,7 +511,8 @@ int chunk_common(qr_kv* kv, int seq_id, int layer, int pos0, int nq, const void*
     }
     float* q32 = reinterpret_cast<float*>(st + ((qbytes + 255) & ~size_t(255)));
     float* dout = out_is_dev ? attn : q32 + nq * rowf;
-    const bool tiles16 = chunk_mfma_eligible(kv->dtype, kv->head_dim, kv->heads, kv->kv_heads);
+    const bool tiles16 = chunk_mfma_eligible(kv->dtype, kv->head_dim, kv->heads, kv->kv_heads) ||
+                         chunk_mfma_split_eligible(kv->dtype, kv->head_dim, kv->heads, kv->kv_heads, pos0, nq);
     if (tiles16 || chunk_f32_eligible(kv->dtype, kv->head_dim, kv->heads, kv->kv_heads, pos0, nq)) {
         // MFMA tiles read each K/V tile once for a block of queries
         ChunkArgs c{};

@@ -192,3 +192,26 @@ def test_chunk_f32_tiles_unseen_infinities(gpu, dtype, heads, kv_heads, D, nq):
     for i in range(bad):
         assert errors(out["inf"][i], out["plain"][i])[1] <= 5e-6, i
     assert np.all(out["inf"][bad:] == np.inf)
+
+
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq,q_dtype", [
+    ("f16", 28, 4, 128, 0, 130, "f16"),      # group 7: 18 queries fill 126 of a block's 128 rows
+    ("bf16", 24, 8, 64, 300, 131, "f32"),    # group 3, hi + lo queries
+    ("bf16", 24, 8, 128, 5000, 9, "bf16"),   # one N tile (position halves), keys split
+    ("f16", 20, 4, 64, 1000, 140, "f32"),    # group 5
+    ("f16", 63, 1, 128, 5, 133, "f16"),      # group 63: one query per block of 64 rows, two of 128
+])
+def test_chunk_mfma_uneven_groups(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dtype):
+    """P (and fp32 queries) in hi + lo parts: about 22 (f16) and 16 (bf16) bits of each product's
+    weight, 2e-5 and 2e-4 relative with the parts' own rounding (2^-16 times a few)."""
+    n = pos0 + nq
+    Kb, Kd, Vb, Vd = make(n + heads, n, kv_heads * D, dtype)
+    qb, qd = to_dtype_bits(np.random.default_rng(n).standard_normal((nq, heads * D), dtype=np.float32), q_dtype)
+    scale = 1 / math.sqrt(D)
+    with qr.PagedKvCache(1, heads, kv_heads, D, n + 10, kv_dtype=dtype) as kv:
+        kv.AppendRange(0, 0, Kb, Vb, src_dtype=dtype)
+        out = kv.AttentionChunk(0, pos0, qb, scale, q_dtype=q_dtype)
+    want = causal_f64(Kd, Vd, qd, heads, kv_heads, D, pos0, scale)
+    for i in range(nq):
+        a, r = errors(out[i], want[i])
+        assert r <= {"f16": 2e-5, "bf16": 2e-4}[dtype], f"query {i}: rel-L2 {r:.2e} max-abs {a:.2e}"
