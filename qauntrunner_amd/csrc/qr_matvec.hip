@@ -1452,7 +1452,10 @@ MvLayout mv_layout(const MatVecArgs& a) {
         L.slab_cols = a.cols;
         const int rbytes = static_cast<int>(row_bytes);
         const int rmax = std::max(1, std::min(kMvMaxRows, kMvThreads * kMvStageBatch * 16 / rbytes));
-        L.R = static_cast<int>(std::max(1LL, std::min<long long>(rmax, a.rows / 1024)));
+        // Q6_K has one item per block, a chain of 256 products, so few rows leave most threads of a
+        // tile idle (4 rows of 16 blocks: 64 of 256): four times the rows, down to 256 tiles (an
+        // 8B layer of one vector 202 -> 172 us, of 2048 columns 123 -> 76)
+        L.R = static_cast<int>(std::max(1LL, std::min<long long>(rmax, a.rows / (a.fmt == QR_FMT_Q6_K ? 256 : 1024))));
         L.stride = (rbytes + 15) / 16 * 16 + 16;
         L.copy_bytes = 16;
         const int nt = a.cols / fs.block * (a.fmt == QR_FMT_Q4_K ? 8 : 1);
