@@ -287,9 +287,10 @@ __device__ __forceinline__ int claim_pages(const PageClaimArgs& a) {
 // One position at a device-side index: page claim, RoPE and append in one workgroup.  The item
 // kernel needs the claim of a launch before it, two launches of one workgroup each (plus V
 // tiles) whose time is their latency: in a captured step of the 8B shape (fp16, 32 + 8 heads of
-// 128) 3.5 and 6.5 us per layer.  Here thread 0 claims while the others read their rows and the
-// cos/sin of the position are computed: 4.9 us (the step of four layers 134.7 -> 125.4).  Items are 8 dims (d .. d + 3 and d + D/2 ..
-// d + D/2 + 3) of a K, q or V head, the arithmetic that of the item kernel.
+// 128) 3.5 and 6.5 us per layer.  Here one thread claims while the others read their rows and
+// the cos/sin of the position are computed: 4.9 us (the step of four layers 134.7 -> 125.4).
+// Items are 8 dims (d .. d + 3 and d + D/2 .. d + D/2 + 3) of a K, q or V head, the arithmetic
+// that of the item kernel.
 constexpr int kRopeStepThreads = 1024;
 template <int IPT>
 __global__ void __launch_bounds__(kRopeStepThreads) rope_step_kernel(const RopeAppendArgs a, const PageClaimArgs c) {
