@@ -318,6 +318,49 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
             }
             lds_barrier();
         }
+        const bool edge = t0 + kTile > unmasked_end || t0 + kTile > t_end;
+        if constexpr (PSPLIT) {
+            // A row must not meet an infinite or NaN V of a position that it does not see (0 x inf
+            // is NaN): the decode entries, which take these groups' smaller calls, read no
+            // position past their own.  Only tiles that reach past the block's first query; V
+            // times zero, one MFMA per operand, shows whether V is finite.  Otherwise (rare) each
+            // such element goes as it is to the outputs of the rows that see it, which no finite
+            // weight changes, and is cleared for the MFMAs.
+            if (edge) {
+                vec8 zero;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) zero[i] = static_cast<T>(0.f);
+                f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < 2 * NDT; ++c)
+                    z = mfma16(*reinterpret_cast<const vec8*>(vt + 1024 * c + 16 * lane), zero, z);
+                // the same in every wave: all read the whole tile
+                if (__builtin_amdgcn_ballot_w64(!((z[0] + z[1]) + (z[2] + z[3]) == 0.f))) {
+                    // halves: only the wave that scores the position adds it
+#pragma unroll 1
+                    for (int k = PS ? 32 * ph : 0; k < (PS ? 32 * ph + 32 : kTile); ++k) {
+#pragma unroll
+                        for (int dt = 0; dt < NDT; ++dt) {
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {  // dim 16 dt + 4 q4 + r
+                                const float v = static_cast<float>(*reinterpret_cast<const T*>(
+                                    vt + SB * (k >> 5) + 1024 * dt + 16 * (16 * ((k >> 3) & 3) + 4 * q4 + r) + 2 * (k & 7)));
+#pragma unroll
+                                for (int j = 0; j < NT; ++j)
+                                    if (!(fabsf(v) < INFINITY) && t0 + k <= min(t_end - 1, pos0 + row_q[j])) acc[j][dt][r] += v;
+                            }
+                            asm volatile("" ::: "memory");  // no registers for all reads at once
+                        }
+                    }
+                    lds_barrier();
+                    for (int c = threadIdx.x; c < kTile * D; c += 64 * WAVES) {
+                        T* e = reinterpret_cast<T*>(const_cast<char*>(vt)) + c;
+                        if (!(fabsf(static_cast<float>(*e)) < INFINITY)) *e = static_cast<T>(0.f);
+                    }
+                    lds_barrier();
+                }
+            }
+        }
 
         // ---- QK (M tiles mt0 .. mt0 + NMT - 1 of the tile)
         const int mt0 = PS ? 2 * ph : 0;
@@ -354,7 +397,7 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
 
         // ---- causal mask and sequence end, only on tiles that reach past the block's
         // first query or the end (wave-uniform, one or two tiles per workgroup)
-        if (t0 + kTile > unmasked_end || t0 + kTile > t_end) {
+        if (edge) {
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
                 const int lim = min(t_end - 1, pos0 + row_q[j]);  // last position row j sees

@@ -215,3 +215,30 @@ def test_chunk_mfma_uneven_groups(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dt
     for i in range(nq):
         a, r = errors(out[i], want[i])
         assert r <= {"f16": 2e-5, "bf16": 2e-4}[dtype], f"query {i}: rel-L2 {r:.2e} max-abs {a:.2e}"
+
+
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq,bad", [
+    ("f16", 24, 8, 64, 0, 133, 70),       # the second of four query blocks, a split per tile
+    ("f16", 28, 4, 128, 0, 140, 138),     # the last block: two queries see it
+    ("bf16", 28, 4, 64, 500, 129, 510),   # the first block, splits of two tiles
+    ("f16", 28, 4, 128, 0, 1200, 600),    # unsplit: masked and unmasked tiles in one workgroup
+    ("bf16", 24, 8, 128, 300, 131, 372),
+    ("f16", 24, 8, 128, 5000, 9, 5004),   # one N tile: two waves per row group, half a tile each
+    ("bf16", 28, 4, 64, 9000, 18, 9001),
+])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_chunk_mfma_uneven_groups_unseen_infinities(gpu, dtype, heads, kv_heads, D, pos0, nq, bad, value):
+    """A V row that is not finite reaches the queries that see its position and no other: those
+    give the same results as without it, within the tolerance of the uneven groups."""
+    n = pos0 + nq
+    Kb, Kd, Vb, Vd = make(n + heads, n, kv_heads * D, dtype)
+    Vi, _ = to_dtype_bits(np.where(np.arange(n)[:, None] == bad, np.float32(value), Vd), dtype)
+    q = np.random.default_rng(4).standard_normal((nq, heads * D), dtype=np.float32)
+    out = {}
+    for name, v in (("plain", Vb), ("bad", Vi)):
+        with qr.PagedKvCache(1, heads, kv_heads, D, n, kv_dtype=dtype) as kv:
+            kv.AppendRange(0, 0, Kb, v, src_dtype=dtype)
+            out[name] = kv.AttentionChunk(0, pos0, q, 1 / math.sqrt(D))
+    for i in range(bad - pos0):
+        assert errors(out["bad"][i], out["plain"][i])[1] <= {"f16": 2e-5, "bf16": 2e-4}[dtype], f"query {i}"
+    assert not np.isfinite(out["bad"][bad - pos0:]).any()
