@@ -30,6 +30,7 @@
 #include "qr_mfma.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace qr {
 namespace {
@@ -80,7 +81,9 @@ struct ChunkK {
     float* out;              // [nq][heads][D]
     float* part_acc;         // [nq*heads][splits][D]
     float2* part_ml;         // [nq*heads][splits]
-    float qscale;            // scale * log2(e)
+    float qscale;            // |scale| log2(e), 1 for scale 0: scores are scaled after the mask and the
+                             // row maximum, so their factor must be positive
+    float qsign;             // sign of scale (0 for scale 0), applied to q
     int queries_per_block;
     int split_tokens;        // multiple of kTile
     int splits;
@@ -259,7 +262,7 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
         amax = max_xor32(amax);
         int qexp = 0;
         if (!BF16 && amax > 16384.f && amax <= 3.0e38f) qexp = static_cast<int>(ceilf(log2f(amax / 16384.f)));
-        const float down = ldexpf(1.f, -qexp);
+        const float down = ldexpf(p.qsign, -qexp);
         sscale[j] = p.qscale * ldexpf(1.f, qexp);
 #pragma unroll
         for (int kk = 0; kk < NK; ++kk)
@@ -667,7 +670,8 @@ hipError_t launch_chunk(const ChunkArgs& a, const ChunkPlan& pl, void* workspace
     const size_t rows = static_cast<size_t>(a.nq) * a.heads;
     k.part_acc = static_cast<float*>(workspace);
     k.part_ml = reinterpret_cast<float2*>(static_cast<char*>(workspace) + rows * pl.splits * a.geom.head_dim * 4);
-    k.qscale = static_cast<float>(static_cast<double>(a.scale) * 1.4426950408889634);
+    k.qscale = a.scale == 0.f ? 1.f : static_cast<float>(std::fabs(static_cast<double>(a.scale)) * 1.4426950408889634);
+    k.qsign = a.scale == 0.f ? 0.f : a.scale < 0.f ? -1.f : 1.f;
     k.queries_per_block = pl.queries_per_block;
     k.split_tokens = pl.split_tokens;
     k.splits = pl.splits;

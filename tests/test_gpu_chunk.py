@@ -242,3 +242,24 @@ def test_chunk_mfma_uneven_groups_unseen_infinities(gpu, dtype, heads, kv_heads,
     for i in range(bad - pos0):
         assert errors(out["bad"][i], out["plain"][i])[1] <= {"f16": 2e-5, "bf16": 2e-4}[dtype], f"query {i}"
     assert not np.isfinite(out["bad"][bad - pos0:]).any()
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.09])
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq,q_dtype", [
+    ("f16", 28, 4, 128, 0, 140, "f16"),
+    ("bf16", 24, 8, 64, 300, 131, "f32"),
+    ("f16", 24, 8, 128, 5000, 9, "f32"),
+    ("bf16", 32, 8, 128, 100, 70, "bf16"),
+    ("f16", 64, 8, 64, 900, 6, "f32"),
+])
+def test_chunk_mfma_scale_zero_and_negative(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dtype, scale):
+    """Scale 0 is the mean of the rows seen so far, a negative one favours the opposite keys."""
+    n = pos0 + nq
+    Kb, Kd, Vb, Vd = make(n + heads, n, kv_heads * D, dtype)
+    qb, qd = to_dtype_bits(np.random.default_rng(n).standard_normal((nq, heads * D), dtype=np.float32), q_dtype)
+    with qr.PagedKvCache(1, heads, kv_heads, D, n, kv_dtype=dtype) as kv:
+        kv.AppendRange(0, 0, Kb, Vb, src_dtype=dtype)
+        out = kv.AttentionChunk(0, pos0, qb, scale, q_dtype=q_dtype)
+    want = causal_f64(Kd, Vd, qd, heads, kv_heads, D, pos0, scale)
+    for i in range(nq):
+        assert errors(out[i], want[i])[1] <= TOL_REL[dtype], f"query {i}"
