@@ -23,8 +23,9 @@
 // PV k-slots of step ks.
 // Operands stay in the cache's 16-bit type (no conversion); q enters as hi + lo parts
 // when its own type is not the cache's (fp32 queries keep ~22 or ~16 bits), P is
-// rounded to the cache type (groups that are not a power of two: hi + lo parts); accumulation and softmax are fp32.  Row sums come from
-// the MFMA too (a ones operand), consistent with the rounded P of the numerator.
+// rounded to the cache type (groups that are not a power of two: hi + lo parts); accumulation
+// and softmax are fp32.  Row sums come from the MFMA too (a ones operand), consistent with the
+// rounded P of the numerator (hi + lo parts: sums of the fp32 weights).
 // The causal mask is applied only on tiles that reach past the block's first query.
 #include "qr_chunk.hpp"
 #include "qr_mfma.hpp"
@@ -134,8 +135,12 @@ __device__ __forceinline__ float max_quarters(float x) {
 
 // BF16: cache element type; NT: 16-row N tiles per wave; NSTAGE: LDS tile buffers;
 // QSPLIT: q is not exact in the cache type and enters as hi + lo parts.
-// PSPLIT: P enters PV as hi + lo parts too (and the row sums are of both), as in the decode
-// kernel that served the shape before.
+// PSPLIT: P enters PV as hi + lo parts too and the row sums add the fp32 weights, as in the
+// decode kernel that served the shape before (fp16 parts drop weights below 2^-25).  For bf16
+// parts the maximum does not lag, so that a row's largest weight is 1 and exact, as it is in each
+// of the decode kernel's waves: with the lag of 2^8 the errors of 24 heads over 8, 1000 queries
+// from scratch were 3.53e-6 from 64 bits (decode entries 3.48e-6, without it 3.40e-6), for 2-6%
+// of the time (24 heads over 8, 24 queries after 20000: 33.4 -> 35.4 us; as entries 160).
 template <bool BF16, int D, int NT, int NSTAGE, bool QSPLIT, bool PSPLIT>
 // Workgroups per CU: two at NT <= 2 with two LDS stages (64 KiB); one with three stages
 // (96 KiB of LDS).  NT = 1 runs eight waves per workgroup.
@@ -154,6 +159,7 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
     constexpr int KI = KB / 1024 / WAVES;    // K DMA instructions per wave and tile
     constexpr int VI = VB / 1024 / WAVES;    // V DMA instructions per wave and tile
     constexpr int PER_TILE = KI + VI;        // vector-memory ops per wave and tile
+    constexpr float kSlack = PSPLIT && BF16 ? 0.f : 8.f;  // log2 units the running max may lag behind
     static_assert(KI >= 1 && VI >= 1, "tile must split over the waves");
 
     __shared__ __attribute__((aligned(1024))) char lds[NSTAGE][KB + VB];
@@ -279,10 +285,11 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
     for (int i = 0; i < 8; ++i) ones[i] = static_cast<T>(1.f);
 
     f32x4_t acc[NT][NDT], accl[NT];
-    float m[NT];
+    float m[NT], ls[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         m[j] = -INFINITY;
+        ls[j] = 0.f;
         accl[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int t = 0; t < NDT; ++t) acc[j][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -416,7 +423,7 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
         }
 
         // ---- online softmax per row: lazy rescale (m moves when the tile max exceeds it
-        // by more than 2^8, so P <= 256), one wave-uniform check for all rows of the lane
+        // by more than 2^kSlack, so P <= 256), one wave-uniform check for all rows of the lane
         float ts[NT];
         bool grow[NT];
         bool any_rescale = false;
@@ -439,14 +446,15 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
                 tmax = max_quarters(max3f(a0, a1, max2f(sc[j][1][2], sc[j][1][3])));
             }
             ts[j] = tmax * sscale[j];
-            grow[j] = ts[j] > m[j] + 8.f;
+            grow[j] = ts[j] > m[j] + kSlack;
             any_rescale |= grow[j] && m[j] != -INFINITY;
         }
         if (__builtin_amdgcn_ballot_w64(any_rescale)) {
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
                 const float corr = grow[j] && m[j] != -INFINITY ? fast_exp2(m[j] - ts[j]) : 1.f;
-                accl[j] *= corr;
+                if (PSPLIT) ls[j] *= corr;
+                else accl[j] *= corr;
 #pragma unroll
                 for (int t = 0; t < NDT; ++t) acc[j][t] *= corr;
             }
@@ -456,15 +464,18 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
         for (int j = 0; j < NT; ++j) {
             if (grow[j]) m[j] = ts[j];
             const float mneg = m[j] == -INFINITY ? 0.f : -m[j];
+            f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int lm = 0; lm < NMT; ++lm)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const float e = fast_exp2(fmaf(sc[j][lm][r], sscale[j], mneg));
+                    if (PSPLIT) sum[r] += e;
                     const T hi = static_cast<T>(e);
                     pb[j][lm >> 1][4 * (lm & 1) + r] = hi;
                     if (PSPLIT) pl[j][lm >> 1][4 * (lm & 1) + r] = static_cast<T>(e - static_cast<float>(hi));
                 }
+            if (PSPLIT) ls[j] += (sum[0] + sum[1]) + (sum[2] + sum[3]);
         }
 
         // ---- PV (and the row sums: a ones operand turns the MFMA into sum over positions).
@@ -479,10 +490,8 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
                 va[dt] = *reinterpret_cast<const vec8*>(vt + SB * ks + 1024 * dt + 16 * lane);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                accl[j] = mfma16(ones, pb[j][kq], accl[j]);
-                if (PSPLIT) accl[j] = mfma16(ones, pl[j][kq], accl[j]);
-            }
+            for (int j = 0; j < NT; ++j)
+                if (!PSPLIT) accl[j] = mfma16(ones, pb[j][kq], accl[j]);
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
@@ -491,6 +500,11 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
                     if (PSPLIT) acc[j][dt] = mfma16(va[dt], pl[j][kq], acc[j][dt]);
                 }
         }
+    }
+
+    if constexpr (PSPLIT) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) accl[j][0] = sum_xor32(sum_xor16(ls[j]));
     }
 
     if constexpr (PS) {

@@ -263,3 +263,23 @@ def test_chunk_mfma_scale_zero_and_negative(gpu, dtype, heads, kv_heads, D, pos0
     want = causal_f64(Kd, Vd, qd, heads, kv_heads, D, pos0, scale)
     for i in range(nq):
         assert errors(out[i], want[i])[1] <= TOL_REL[dtype], f"query {i}"
+
+
+def test_chunk_mfma_uneven_groups_sum_small_weights(gpu):
+    """Row sums of uneven groups are of the fp32 weights: position 0 has weight 1 and each of up
+    to 4,143 others 2^-25.2, which fp16 hi + lo parts drop (below half of 2^-24) although they
+    add up to 1.1e-4.  V cancels but at position 0, so the output is that row over the sum."""
+    heads, kv_heads, D, pos0, nq = 24, 8, 64, 2800, 1344  # keys unsplit
+    n = pos0 + nq
+    K = np.zeros((n, kv_heads * D), np.float32)
+    K[0] = np.float16(25.2 * math.log(2) / 8)  # score 8 K log2(e) log2 units above the others
+    V = np.where(np.arange(n)[:, None] % 2 == 0, np.float32(1), np.float32(-1)) * np.ones((1, kv_heads * D), np.float32)
+    Kb, Kd = to_dtype_bits(K, "f16")
+    Vb, Vd = to_dtype_bits(V, "f16")
+    q = np.ones((nq, heads * D), np.float32)
+    with qr.PagedKvCache(1, heads, kv_heads, D, n, kv_dtype="f16") as kv:
+        kv.AppendRange(0, 0, Kb, Vb, src_dtype="f16")
+        out = kv.AttentionChunk(0, pos0, q, 1 / 8)
+    want = causal_f64(Kd, Vd, q, heads, kv_heads, D, pos0, 1 / 8)
+    for i in range(nq):
+        assert errors(out[i], want[i])[1] <= 2e-5, f"query {i}"
