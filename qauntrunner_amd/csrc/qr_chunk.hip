@@ -74,6 +74,7 @@ struct ChunkK {
     int kv_heads;
     int heads;
     int group;
+    int group_shift;         // log2(group) where that is whole
     int pos0;
     const int* pos0_dev;     // device position of query 0 (clamped to [0, pos0]) when set
     int nq;
@@ -197,9 +198,9 @@ __global__ void __launch_bounds__(NT == 1 ? 512 : 256, NT <= 2 && NSTAGE <= 2 ? 
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         const int rho = rw * 16 * NT + j * 16 + col;
-        const int dq = rho / p.group;
+        const int dq = PSPLIT ? rho / p.group : rho >> p.group_shift;
         row_q[j] = q_first + dq;
-        row_h[j] = kvh * p.group + (rho - dq * p.group);
+        row_h[j] = kvh * p.group + (PSPLIT ? rho - dq * p.group : rho & (p.group - 1));
         row_on[j] = row_q[j] < p.nq && dq < p.queries_per_block;
     }
     const int q_last = min(p.nq, q_first + p.queries_per_block) - 1;
@@ -675,6 +676,7 @@ hipError_t launch_chunk(const ChunkArgs& a, const ChunkPlan& pl, void* workspace
     k.heads = a.heads;
     k.group = a.heads / a.geom.kv_heads;
     const bool psplit = (k.group & (k.group - 1)) != 0;
+    while ((2 << k.group_shift) <= k.group) ++k.group_shift;
     k.pos0 = a.pos0;
     k.pos0_dev = a.pos0_dev;
     k.nq = a.nq;
