@@ -41,7 +41,6 @@ namespace qr {
 namespace {
 
 constexpr int kTP = 32;               // positions per tile
-constexpr float kSlack = 8.f;         // log2 units the running max may lag behind (P <= 256)
 
 struct ChunkF32K {
     const char* pool;
@@ -303,14 +302,15 @@ __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f3
             bad = __builtin_amdgcn_ballot_w64(bad) != 0;
         }
 
-        // ---- online softmax (lazy rescale)
+        // ---- online softmax.  The maximum does not lag, so that P <= 1 as in the decode kernels: a V
+        // of more than 2^120 would overflow under P <= 256.
         float tm = -INFINITY;
 #pragma unroll
         for (int mt = 0; mt < NMT; ++mt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) tm = fmaxf(tm, sc[mt][r]);
         tm = max_xor32(max_xor16(tm));
-        const bool grow = tm > m + kSlack;
+        const bool grow = tm > m;
         const bool rescale = grow && m != -INFINITY;
         if (__builtin_amdgcn_ballot_w64(rescale)) {
             const float corr = rescale ? fast_exp2(m - tm) : 1.f;

@@ -194,6 +194,25 @@ def test_chunk_f32_tiles_unseen_infinities(gpu, dtype, heads, kv_heads, D, nq):
     assert np.all(out["inf"][bad:] == np.inf)
 
 
+@pytest.mark.parametrize("dtype,heads,kv_heads,D", [("f32", 8, 2, 64), ("f32", 16, 16, 128), ("f32", 16, 16, 256),
+                                                     ("bf16", 24, 8, 96)])
+def test_chunk_f32_tiles_large_values(gpu, dtype, heads, kv_heads, D):
+    """V near the top of the range.  Positions 0 to 31 have score 0, position 40 one of 7.5 log2
+    units above and the others none to speak of, so a weight against any earlier maximum would
+    overflow (2^7.5 x 5e36) where weights of at most 1 add up to 33 at most (1.7e38)."""
+    nq, scale, v = 66, 1 / math.sqrt(D), 5e36
+    K = np.full((nq, kv_heads * D), -100 / (D * scale), np.float32)
+    K[:32] = 0
+    K[40] = 7.5 * math.log(2) / (D * scale)
+    Kb, _ = to_dtype_bits(K, dtype)
+    Vb, Vd = to_dtype_bits(np.full((nq, kv_heads * D), v, np.float32), dtype)
+    q = np.ones((nq, heads * D), np.float32)
+    with qr.PagedKvCache(1, heads, kv_heads, D, nq, kv_dtype=dtype) as kv:
+        kv.AppendRange(0, 0, Kb, Vb, src_dtype=dtype)
+        out = kv.AttentionChunk(0, 0, q, scale)
+    assert np.all(np.abs(out / Vd[0, 0] - 1) <= 5e-6)  # the fp32 sums' bound of the tests above
+
+
 @pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq,q_dtype", [
     ("f16", 28, 4, 128, 0, 130, "f16"),      # group 7: 18 queries fill 126 of a block's 128 rows
     ("bf16", 24, 8, 64, 300, 131, "f32"),    # group 3, hi + lo queries
