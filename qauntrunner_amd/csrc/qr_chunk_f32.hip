@@ -12,7 +12,7 @@
 // at that rate) took 8 launches of 61 us, 506 us per call with the append; this kernel takes 152
 // and its merge 7 (157 per call).  The matrix units are busy 81% of the cycles in which waves
 // are resident (1.0 LDS conflict cycle per MFMA); the rest is the softmax and the tile barriers.
-// Error against 64-bit results there: 3.3e-7 (decode entries 3.1e-7).
+// Error against 64-bit results there: 2.9e-7 (decode entries 3.15e-7).
 //
 // A row is one (query, query head) pair.  Workgroup = 4 waves; the K/V tile of 32 positions is
 // copied into LDS by buffer-load DMA (two stages) and serves 64 / PG rows:
@@ -27,9 +27,13 @@
 //   PV  O^T[dim][row]: lane quarter q4 holds the scores of positions 4q4 + r; step r takes
 //       those four positions as its k-slots, so P enters from the lane's own registers.  A is
 //       V row 4q4 + r, PE consecutive dims per lane: one LDS read feeds PE MFMAs.
-// Sums are blocked -- 16 or 32 dims of a score, one tile's positions of an output are summed
-// from zero and then added -- so that an fp32 MFMA chain is no longer than the decode
-// kernels' (one chain over 512 positions: 9.5e-7 from 64-bit results against 3.1e-7).
+// Sums are blocked, because an fp32 MFMA chain rounds at the size of its running sum (one chain
+// over 512 positions: 9.5e-7 from 64-bit results where the decode entries have 3.1e-7).  A score is
+// chains of two MFMAs (8 dims), added in pairs and then to the sum of the even or the odd steps;
+// an output adds chains of two MFMAs (8 positions; four for 16-bit head_dim 256) in pairs before
+// they go to the accumulator.  Distance from 64-bit results, decode entries and here: 3.15e-7 and
+// 2.92e-7 at the shape above, 1.85e-7 and 1.84e-7 for 1000 queries from scratch (chains of four
+// and eight MFMAs: 3.34e-7 and 2.25e-7; chains of one and two 2.90e-7 and 1.83e-7, 7% slower).
 // 16-byte chunk c of an LDS row r sits at c ^ (r & SW): the 16 rows that a QK read takes lie a
 // multiple of 128 bytes apart.
 #include "qr_chunk.hpp"
@@ -118,6 +122,16 @@ template <typename ST, int N> struct Elems {
     static constexpr int kWords = std::is_same<ST, float>::value ? N : N / 2;
     typedef uint32_t type __attribute__((ext_vector_type(kWords)));
     __device__ static __forceinline__ type read(const char* p) { return *reinterpret_cast<const type*>(p); }
+    // a pair with the elements that are not kept cleared
+    __device__ static __forceinline__ type keep(type w, bool k0, bool k1) {
+        if constexpr (std::is_same<ST, float>::value) {
+            if (!k0) w[0] = 0;
+            if (!k1) w[1] = 0;
+        } else {
+            w[0] &= (k0 ? 0xFFFFu : 0u) | (k1 ? 0xFFFF0000u : 0u);
+        }
+        return w;
+    }
     __device__ static __forceinline__ void widen(const type w, float (&o)[N]) {
         if constexpr (std::is_same<ST, float>::value) {
 #pragma unroll
@@ -137,6 +151,13 @@ template <typename ST, int N> struct Elems {
         }
     }
 };
+
+// Sum of 1, 2 or 4 chains, pairwise.
+template <int N> __device__ __forceinline__ f32x4_t chain_sum(const f32x4_t (&c)[N]) {
+    if constexpr (N == 1) return c[0];
+    else if constexpr (N == 2) return c[0] + c[1];
+    else return (c[0] + c[1]) + (c[2] + c[3]);
+}
 
 template <typename ST, int D, int PG>
 __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f32_kernel(const ChunkF32K p) {
@@ -249,8 +270,16 @@ __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f3
         // partial sums are added during step jj + 1
         f32x4_t sc[NMT];
         {
+            constexpr int NC = EPC / 2;  // chains of two MFMAs
             U32x4 raw[2][NMT];
-            f32x4_t part[2][NMT];
+            f32x4_t part[2][NMT][NC], sum[2][NMT];
+            auto add = [&](int jj) __attribute__((always_inline)) {  // step jj's chains to the sum of its parity
+#pragma unroll
+                for (int mt = 0; mt < NMT; ++mt) {
+                    const f32x4_t s = chain_sum<NC>(part[jj & 1][mt]);
+                    sum[jj & 1][mt] = jj < 2 ? s : sum[jj & 1][mt] + s;
+                }
+            };
             auto kread = [&](int jj) __attribute__((always_inline)) {
 #pragma unroll
                 for (int mt = 0; mt < NMT; ++mt) raw[jj & 1][mt] = load16(base + kx[jj & 1] + 128 * (jj >> 1) + 16 * mt * RB);
@@ -264,23 +293,26 @@ __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f3
 #pragma unroll
                 for (int mt = 0; mt < NMT; ++mt) {
                     Chunk<ST>::widen(raw[jj & 1][mt], kv[mt]);
-                    part[jj & 1][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) part[jj & 1][mt][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
                 }
 #pragma unroll
-                for (int e = 0; e < EPC; ++e)
+                for (int e = 0; e < EPC; ++e) {
+                    if (jj > 0 && e == EPC / 2) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        add(jj - 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
 #pragma unroll
                     for (int mt = 0; mt < NMT; ++mt)
-                        part[jj & 1][mt] =
-                            __builtin_amdgcn_mfma_f32_16x16x4f32(kv[mt][e], qv[jj][e], part[jj & 1][mt], 0, 0, 0);
-#pragma unroll
-                for (int mt = 0; mt < NMT; ++mt) {
-                    if (jj == 1) sc[mt] = part[0][mt];
-                    if (jj > 1) sc[mt] += part[(jj - 1) & 1][mt];
+                        part[jj & 1][mt][e % NC] =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(kv[mt][e], qv[jj][e], part[jj & 1][mt][e % NC], 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
+            add(NJ - 1);
 #pragma unroll
-            for (int mt = 0; mt < NMT; ++mt) sc[mt] += part[(NJ - 1) & 1][mt];
+            for (int mt = 0; mt < NMT; ++mt) sc[mt] = sum[0][mt] + sum[1][mt];
         }
 
         // ---- causal mask, only on tiles that reach past the block's first query (the keys'
@@ -293,13 +325,16 @@ __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f3
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     sc[mt][r] = t0 + half0 + 16 * mt + 4 * q4 + r <= row_lim ? sc[mt][r] : -INFINITY;
-            for (int c = lane; c < NMT * 16 * NCH; c += 64) {
+            // the whole tile, so that every wave finds the same; V times zero is zero or NaN
+            float z = 0.f;
+#pragma unroll 4
+            for (int i = 0; i < kTP * NCH / 64; ++i) {
                 float v[EPC];
-                Chunk<ST>::widen(load16(base + KB + half0 * RB + 16 * c), v);
+                Chunk<ST>::widen(load16(base + KB + 16 * (lane + 64 * i)), v);
 #pragma unroll
-                for (int e = 0; e < EPC; ++e) bad |= !(fabsf(v[e]) < INFINITY);
+                for (int e = 0; e < EPC; ++e) z = fmaf(v[e], 0.f, z);
             }
-            bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+            bad = __builtin_amdgcn_ballot_w64(!(z == 0.f)) != 0;
         }
 
         // ---- online softmax.  The maximum does not lag, so that P <= 1 as in the decode kernels: a V
@@ -331,9 +366,10 @@ __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f3
         for (int mt = 1; mt < NMT; ++mt) ls += sc[mt];
         l += (ls[0] + ls[1]) + (ls[2] + ls[3]);
 
-        if (edge && bad) {
-            // A row must not meet the V of a position that it does not see: 0 x inf is NaN.
-            // One position at a time, added only where the row sees it (rare: V holds inf/NaN).
+        if (bad) {
+            // A row must not meet the V of a position that it does not see: 0 x inf is NaN.  The
+            // elements that are not finite are added here, only where the row sees their position
+            // (rare), and cleared for the products below.
 #pragma unroll 1
             for (int k = 0; k < NMT * 16; ++k) {  // position 16 (k / 16) + 4 ((k / 4) % 4) + k % 4
                 const int pos = half0 + k;
@@ -352,16 +388,30 @@ __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f3
                         float v[PE];
                         El::widen(El::read(base + KB + pos * RB + 16 * ((b >> 4) ^ (pos & SW)) + (b & 15)), v);
 #pragma unroll
-                        for (int e = 0; e < PE; ++e) acc[g][e][rr] = see ? fmaf(w, v[e], acc[g][e][rr]) : acc[g][e][rr];
+                        for (int e = 0; e < PE; ++e)
+                            if (see && !(fabsf(v[e]) < INFINITY)) acc[g][e][rr] = fmaf(w, v[e], acc[g][e][rr]);
                         asm volatile("" ::: "memory");  // no registers for all reads at once
                     }
                 }
             }
-            continue;
+            lds_barrier();  // every wave has read them
+            for (int c = threadIdx.x; c < kTP * NCH; c += 256) {
+                typedef typename Elems<ST, 2>::type Pair;
+#pragma unroll
+                for (int i = 0; i < EPC / 2; ++i) {
+                    Pair* const w = reinterpret_cast<Pair*>(const_cast<char*>(base) + KB + 16 * c) + i;
+                    float v[2];
+                    Elems<ST, 2>::widen(*w, v);
+                    const bool b0 = !(fabsf(v[0]) < INFINITY), b1 = !(fabsf(v[1]) < INFINITY);
+                    if (b0 || b1) *w = Elems<ST, 2>::keep(*w, !b0, !b1);
+                }
+            }
+            lds_barrier();
         }
 
         // ---- weighted sum of V (step st = 4 mt + r of dim group g; V read two steps ahead)
-        constexpr int NS = 4 * NMT;
+        constexpr int CL = D == 256 && EPC == 8 ? 4 : 2;  // steps of a chain
+        constexpr int NS = 4 * NMT, NC = NS / CL, NO = NC + 1;
         typename El::type vb[3];
         auto vread = [&](int i) __attribute__((always_inline)) {
             const int g = i / NS, st = i % NS;
@@ -369,30 +419,37 @@ __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f3
         };
         vread(0);
         vread(1);
-        f32x4_t o[2][PE];
+        f32x4_t o[NO][PE];  // chain c of group g in o[(NC g + c) % NO]: the next group's first chain leaves g's alone
+        auto add = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = 0; e < PE; ++e) {
+                f32x4_t s[NC];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) s[c] = o[(NC * g + c) % NO][e];
+                acc[g][e] += chain_sum<NC>(s);
+            }
+        };
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
 #pragma unroll
-            for (int e = 0; e < PE; ++e) o[g & 1][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
             for (int st = 0; st < NS; ++st) {
-                const int i = NS * g + st;
+                const int i = NS * g + st, c = i / CL % NO;
+                if (st % CL == 0) {
+#pragma unroll
+                    for (int e = 0; e < PE; ++e) o[c][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                }
                 if (i + 2 < NS * NG) vread(i + 2);
                 __builtin_amdgcn_sched_barrier(0);
                 float v[PE];
                 El::widen(vb[i % 3], v);
 #pragma unroll
                 for (int e = 0; e < PE; ++e)
-                    o[g & 1][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], sc[st >> 2][st & 3], o[g & 1][e], 0, 0, 0);
-                if (g > 0 && st == 1) {
-#pragma unroll
-                    for (int e = 0; e < PE; ++e) acc[g - 1][e] += o[(g - 1) & 1][e];
-                }
+                    o[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], sc[st >> 2][st & 3], o[c][e], 0, 0, 0);
+                if (g > 0 && st == 1) add(g - 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-#pragma unroll
-        for (int e = 0; e < PE; ++e) acc[NG - 1][e] += o[(NG - 1) & 1][e];
+        add(NG - 1);
     }
     l = sum_xor32(sum_xor16(l));
 
@@ -435,7 +492,12 @@ __global__ void __launch_bounds__(256, (F32Geom<ST, D>::wg_per_cu(PG))) chunk_f3
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int e = 0; e < PE; ++e) o[16 * PE * g + PE * r + e] = acc[g][e][r] * by;
+            for (int e = 0; e < PE; ++e) {
+                const float a = acc[g][e][r];
+                float x = a * by;
+                if (p.splits == 1 && fabsf(x) < INFINITY) x = fmaf(fmaf(-x, l, a), by, x);  // a / l to the last bit or so
+                o[16 * PE * g + PE * r + e] = x;
+            }
     if (p.splits > 1 && q4 == 0) p.part_ml[slot] = make_float2(m, l);
 }
 

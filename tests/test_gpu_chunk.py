@@ -194,6 +194,32 @@ def test_chunk_f32_tiles_unseen_infinities(gpu, dtype, heads, kv_heads, D, nq):
     assert np.all(out["inf"][bad:] == np.inf)
 
 
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq", [
+    ("f32", 16, 4, 64, 0, 500),
+    ("f32", 32, 8, 128, 0, 300),
+    ("f32", 32, 8, 128, 1000, 200),
+    ("f32", 16, 16, 256, 0, 300),
+    ("bf16", 24, 8, 96, 0, 300),
+    ("f16", 32, 8, 256, 0, 300),
+])
+def test_chunk_f32_tiles_error_of_decode_entries(gpu, dtype, heads, kv_heads, D, pos0, nq):
+    """The distance from 64-bit results is no larger than that of one decode entry per query: 5%
+    for the spread from seed to seed (1 to 3% over three seeds of these shapes)."""
+    n = pos0 + nq
+    Kb, Kd, Vb, Vd = make(n + heads, n, kv_heads * D, dtype)
+    q = np.random.default_rng(n).standard_normal((nq, heads * D), dtype=np.float32) * np.float32(1.5)
+    scale = 1 / math.sqrt(D)
+    with qr.PagedKvCache(1, heads, kv_heads, D, n, kv_dtype=dtype) as kv:
+        kv.AppendRange(0, 0, Kb, Vb, src_dtype=dtype)
+        tiles = kv.AttentionChunk(0, pos0, q, scale)
+        entries = np.concatenate([kv.AttentionBatch(0, [0] * len(r), list(r), q[r.start - pos0:r.stop - pos0], scale)
+                                  for r in (range(p, min(p + 64, n)) for p in range(pos0, n, 64))])
+    want = causal_f64(Kd, Vd, q, heads, kv_heads, D, pos0, scale)
+    a, b = (np.linalg.norm(x.reshape(want.shape) - want) / np.linalg.norm(want) for x in (tiles, entries))
+    print(f"tiles {a:.3e} entries {b:.3e}")
+    assert a <= 1.05 * b
+
+
 @pytest.mark.parametrize("dtype,heads,kv_heads,D", [("f32", 8, 2, 64), ("f32", 16, 16, 128), ("f32", 16, 16, 256),
                                                      ("bf16", 24, 8, 96)])
 def test_chunk_f32_tiles_large_values(gpu, dtype, heads, kv_heads, D):
