@@ -608,23 +608,39 @@ ChunkPlan plan_chunk_f32(const ChunkArgs& a) {
     const int tiles = (a.pos0 + a.nq + kTP - 1) / kTP;
     ChunkPlan best{};
     double best_cost = 0;
-    // Position halves and splits of the keys by the time of the matrix work (a tile of 16 rows
-    // and 32 positions is 2048 D / 64 cycles of a SIMD, shared by the resident waves) plus the
-    // partials' traffic (written and read once, about 4 TB/s) and the merge's launch.  At the
-    // shape above: 64 rows in 2 splits 152 + 7 us (kernel + merge), in 1 split 184, in 4 158 + 8;
-    // position halves 165 in 1 split (8% more per tile: a barrier per half the work).
+    // Position halves and splits of the keys by the time of the matrix work plus the partials'
+    // traffic (written and read once, about 4 TB/s) and the merge's launch.  A tile of 64 rows and
+    // 32 positions is 32 D cycles of a CU's matrix units; with w workgroups resident a tile of each
+    // takes 0.8 (w + 1) of that (a workgroup alone leaves the units idle in its softmax and
+    // barriers, several overlap), position halves 0.65 of it instead of a half (a barrier per half
+    // the work).  Query blocks of like lengths (many keys before them) run in whole rounds of the
+    // longest; blocks from scratch mix, so they take the mean length.  Over 163 shapes the choice
+    // took 2.6% more than the fastest of up to ten (by whole occupancy rounds alone 7.9%).  At the
+    // shape above 64 rows in 1, 2, 3 and 4 splits 193, 158, 195 and 164 us with the append, halves in
+    // 1 and 2 163 and 177; 1059 queries from scratch at head_dim 64: 64 rows 91, halves 68; 512 after
+    // 1536 at head_dim 256 in 16 bits: 64 rows 468, halves 346.
+    // Splits are for units that leave CUs idle: no more of them than fill the CUs four times over,
+    // which bounds the partials too (4 x 768 workgroups x 64 rows of head_dim 96: 77 MB).
+    const int cus = cu_count();
+    const double like = static_cast<double>(a.pos0) / (a.pos0 + a.nq);  // 0 from scratch
+    auto tile_cost = [](double w) { return 0.8 * (w + 1.0); };
     for (int pg = 1; pg <= 2; ++pg) {
-        const int per_cu = wgs_per_cu(a.kv_dtype, D, pg), slots = cu_count() * per_cu;
+        const int per_cu = wgs_per_cu(a.kv_dtype, D, pg), slots = cus * per_cu;
         const int wg_rows = 64 / pg;
         if (wg_rows < g) continue;
         const int qpb = wg_rows / g, qblocks = (a.nq + qpb - 1) / qpb;
         const long long units = static_cast<long long>(qblocks) * a.geom.kv_heads;
-        const double tile_us = 32.0 * D / 2400 * per_cu * (pg == 2 ? 0.54 : 1.0);
+        const double tile_us = 32.0 * D / 2400 * (pg == 2 ? 0.65 : 1.0);
         const int smax = std::min(64, std::max(1, tiles / 4));
-        for (int s = 1; s <= smax; ++s) {
-            const long long rounds = (units * s + slots - 1) / slots;
+        for (int s = 1; s <= smax && (s == 1 || units * s <= 4LL * slots); ++s) {
+            const long long full = units * s / slots, rest = units * s % slots;
+            const double longest = (tiles + s - 1) / s + 1.0;
+            const double mean = (a.pos0 + 0.5 * a.nq) / kTP / s + 1.0;
+            const double per = static_cast<double>(units) * s / cus, w = std::min<double>(per_cu, std::max(1.0, per));
+            const double rounds = (full * tile_cost(per_cu) + (rest ? tile_cost((rest + cus - 1) / cus) : 0.0)) * longest;
+            const double mixed = std::max(longest * tile_cost(1), per * mean * tile_cost(w) / w);
             const double traffic = s > 1 ? 5.0 + static_cast<double>(rows) * s * D * 8 / 4e6 : 0.0;
-            const double cost = rounds * ((tiles + s - 1) / s + 1.0) * tile_us + traffic;
+            const double cost = (like * rounds + (1.0 - like) * mixed) * tile_us + traffic;
             if (best.splits == 0 || cost < best_cost) {
                 best_cost = cost;
                 best.nt = 1;

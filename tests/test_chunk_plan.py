@@ -1,0 +1,54 @@
+"""Host-side plans of the fp32 chunk tiles: the split partials stay bounded (CPU only)."""
+import ctypes
+import os
+
+import pytest
+
+from qauntrunner_amd import _lib
+
+
+class Geom(ctypes.Structure):  # PageGeom
+    _fields_ = [("planes", ctypes.c_int), ("kv_heads", ctypes.c_int), ("head_dim", ctypes.c_int), ("mfma", ctypes.c_int)]
+
+
+class Args(ctypes.Structure):  # ChunkArgs
+    _fields_ = [("pool", ctypes.c_void_p), ("page_table", ctypes.c_void_p), ("geom", Geom), ("kv_dtype", ctypes.c_int),
+                ("heads", ctypes.c_int), ("pos0", ctypes.c_int), ("pos0_dev", ctypes.c_void_p), ("nq", ctypes.c_int),
+                ("q", ctypes.c_void_p), ("q_dtype", ctypes.c_int), ("out", ctypes.c_void_p), ("scale", ctypes.c_float)]
+
+
+class Plan(ctypes.Structure):  # ChunkPlan
+    _fields_ = [(f, ctypes.c_int) for f in ("nt", "pg", "queries_per_block", "qblocks", "splits", "split_tokens")] + \
+               [("workspace_bytes", ctypes.c_size_t)]
+
+
+def plan(dtype, heads, kv_heads, D, pos0, nq):
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    f = getattr(ctypes.CDLL(_lib.LIB_PATH), "_ZN2qr14plan_chunk_f32ERKNS_9ChunkArgsE")
+    f.restype, f.argtypes = Plan, [ctypes.POINTER(Args)]
+    a = Args()
+    a.geom.planes, a.geom.kv_heads, a.geom.head_dim = 2, kv_heads, D
+    a.kv_dtype, a.heads, a.pos0, a.nq = dtype, heads, pos0, nq
+    p = f(ctypes.byref(a))
+    assert p.splits == 1 or p.workspace_bytes == nq * heads * p.splits * (4 * D + 8)
+    assert p.qblocks * p.queries_per_block >= nq and (64 // p.pg) // (heads // kv_heads) == p.queries_per_block
+    return p
+
+
+@pytest.mark.parametrize("dtype,D", [(0, 64), (0, 96), (0, 128), (0, 256), (1, 96), (2, 256)])
+def test_chunk_f32_partials_are_bounded(dtype, D):
+    """Long prompts of any length need less than 80 MB of split partials."""
+    for heads, kv_heads in ((8, 2), (16, 16), (28, 4), (32, 8), (64, 8), (64, 1)):
+        for nq in [65, 128, 333, 512, 1000, 4095, 4096, 4097, 5000, 20000] + list(range(1500, 1600, 7)):
+            for pos0 in (0, 1536, 100000):
+                assert plan(dtype, heads, kv_heads, D, pos0, nq).workspace_bytes < 80e6, (heads, kv_heads, nq, pos0)
+
+
+def test_chunk_f32_plans_of_measured_shapes():
+    """The faster form where the forms were timed: 64 rows in two splits (158 us against 163 as
+    position halves), position halves (33 against 38 and more), 64 rows in nine splits (88 against 94 and more), position
+    halves for 16-bit head_dim 256 (346 against 458)."""
+    got = [(p.pg, p.splits) for p in (plan(0, 32, 8, 128, 1536, 512), plan(0, 32, 8, 128, 0, 333),
+                                      plan(0, 32, 8, 128, 4000, 100), plan(1, 32, 8, 256, 1536, 512))]
+    assert got == [(1, 2), (2, 1), (1, 9), (2, 1)]

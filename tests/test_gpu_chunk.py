@@ -153,12 +153,22 @@ def causal_f64(K, V, q, heads, kv_heads, D, pos0, scale):
     ("f32", 24, 8, 96, 1000, 200, "f32"),    # group 3, head_dim 96 (8-byte V reads)
     ("f32", 16, 16, 256, 300, 67, "f16"),    # group 1, head_dim 256
     ("f32", 64, 1, 64, 7, 66, "f32"),        # 64 heads on one kv head
-    ("f32", 32, 8, 64, 700, 600, "f32"),     # two N tiles
+    ("f32", 32, 8, 64, 700, 600, "f32"),     # 64 rows a workgroup (no position halves), keys split
     ("f16", 24, 8, 96, 500, 130, "f16"),     # 16-bit pages, token-major
     ("bf16", 32, 8, 96, 90, 40, "f32"),
     ("bf16", 64, 8, 256, 250, 70, "bf16"),
     ("f16", 8, 2, 256, 9000, 7, "f32"),
     ("f32", 32, 8, 128, 3000, 5, "f32"),     # 20 rows over split keys, from the byte line up
+    # groups above 32: always 64 rows a workgroup, one query each
+    ("f32", 48, 1, 96, 0, 70, "f32"),        # unsplit
+    ("f32", 40, 1, 128, 900, 70, "f32"),     # split
+    ("f32", 64, 1, 128, 0, 100, "bf16"),
+    ("f32", 64, 1, 256, 0, 66, "f32"),
+    ("f32", 33, 1, 256, 2000, 20, "f32"),
+    ("bf16", 64, 1, 96, 30, 40, "bf16"),
+    ("f16", 40, 1, 256, 3000, 75, "f32"),
+    ("f32", 24, 8, 256, 1000, 300, "f32"),   # 64 rows of 21 queries, split
+    ("f32", 32, 8, 128, 700, 300, "f32"),
 ])
 def test_chunk_f32_tiles(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dtype):
     """fp32 arithmetic over the exactly decoded cache: fp32 sums over up to 5,000 keys, 5e-6
@@ -176,8 +186,12 @@ def test_chunk_f32_tiles(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dtype):
         assert r <= 5e-6, f"query {i}: rel-L2 {r:.2e} max-abs {a:.2e}"
 
 
-@pytest.mark.parametrize("dtype,heads,kv_heads,D,nq", [("f32", 8, 2, 64, 70), ("f32", 8, 2, 128, 100), ("bf16", 8, 4, 96, 40),
-                                                         ("f16", 8, 8, 256, 75)])
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,nq", [
+    ("f32", 8, 2, 64, 70), ("f32", 8, 2, 128, 100), ("bf16", 8, 4, 96, 40), ("f16", 8, 8, 256, 300),
+    # 64 rows a workgroup: unsplit, and split
+    ("f32", 64, 1, 96, 70), ("f32", 40, 1, 128, 100), ("f32", 33, 1, 256, 75), ("f16", 64, 1, 96, 300),
+    ("f32", 32, 8, 64, 600), ("bf16", 40, 1, 256, 290),
+])
 def test_chunk_f32_tiles_unseen_infinities(gpu, dtype, heads, kv_heads, D, nq):
     """An infinite V reaches the queries that see its position and no other."""
     Kb, Kd, Vb, Vd = make(3, nq, kv_heads * D, dtype)
