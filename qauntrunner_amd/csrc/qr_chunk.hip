@@ -654,6 +654,10 @@ ChunkPlan plan_chunk(const ChunkArgs& a) {
     // split the keys when there are too few (query block, kv head) units to fill the GPU
     int splits = 1;
     if (units < cu_total()) splits = std::min((cu_total() + units - 1) / units, (total + kTile - 1) / kTile);
+    if (g & (g - 1)) {
+        const size_t each = static_cast<size_t>(a.nq) * a.heads * (static_cast<size_t>(a.geom.head_dim) * 4 + 8);
+        while (splits > 1 && splits * each > a.room) --splits;
+    }
     int split_tokens = ((total + splits - 1) / splits + kTile - 1) / kTile * kTile;
     splits = (total + split_tokens - 1) / split_tokens;
     pl.splits = splits;

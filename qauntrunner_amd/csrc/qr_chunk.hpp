@@ -20,6 +20,9 @@ struct ChunkArgs {
     int q_dtype;
     float* out;             // device [nq][heads][head_dim]
     float scale;
+    // bytes that the split partials may take; the plans that came after the decode entries (fp32
+    // tiles, groups that are not a power of two) use fewer splits when it is less than they want
+    size_t room = ~size_t(0);
 };
 
 struct ChunkPlan {

@@ -632,7 +632,8 @@ ChunkPlan plan_chunk_f32(const ChunkArgs& a) {
         const long long units = static_cast<long long>(qblocks) * a.geom.kv_heads;
         const double tile_us = 32.0 * D / 2400 * (pg == 2 ? 0.65 : 1.0);
         const int smax = std::min(64, std::max(1, tiles / 4));
-        for (int s = 1; s <= smax && (s == 1 || units * s <= 4LL * slots); ++s) {
+        auto bytes = [&](int s) { return static_cast<size_t>(rows) * s * (static_cast<size_t>(D) * 4 + 8); };
+        for (int s = 1; s <= smax && (s == 1 || (units * s <= 4LL * slots && bytes(s) <= a.room)); ++s) {
             const long long full = units * s / slots, rest = units * s % slots;
             const double longest = (tiles + s - 1) / s + 1.0;
             const double mean = (a.pos0 + 0.5 * a.nq) / kTP / s + 1.0;

@@ -527,6 +527,9 @@ int chunk_common(qr_kv* kv, int seq_id, int layer, int pos0, int nq, const void*
         c.q_dtype = q_dtype;
         c.out = dout;
         c.scale = scale;
+        // a captured call cannot grow the workspace: it splits as far as the present one allows,
+        // so that a call made outside capture before it need not have wanted as many splits
+        if (capturing(stream)) c.room = kv->workspace.size();
         const ChunkPlan plan = tiles16 ? plan_chunk(c) : plan_chunk_f32(c);
         QR_TRY(grow_workspace(kv, plan.workspace_bytes, stream));
         QR_HIP(tiles16 ? launch_chunk(c, plan, kv->workspace.get(), stream, kv->split_event)

@@ -14,7 +14,8 @@ class Geom(ctypes.Structure):  # PageGeom
 class Args(ctypes.Structure):  # ChunkArgs
     _fields_ = [("pool", ctypes.c_void_p), ("page_table", ctypes.c_void_p), ("geom", Geom), ("kv_dtype", ctypes.c_int),
                 ("heads", ctypes.c_int), ("pos0", ctypes.c_int), ("pos0_dev", ctypes.c_void_p), ("nq", ctypes.c_int),
-                ("q", ctypes.c_void_p), ("q_dtype", ctypes.c_int), ("out", ctypes.c_void_p), ("scale", ctypes.c_float)]
+                ("q", ctypes.c_void_p), ("q_dtype", ctypes.c_int), ("out", ctypes.c_void_p), ("scale", ctypes.c_float),
+                ("room", ctypes.c_size_t)]
 
 
 class Plan(ctypes.Structure):  # ChunkPlan
@@ -22,17 +23,19 @@ class Plan(ctypes.Structure):  # ChunkPlan
                [("workspace_bytes", ctypes.c_size_t)]
 
 
-def plan(dtype, heads, kv_heads, D, pos0, nq):
+def plan(dtype, heads, kv_heads, D, pos0, nq, room=2**64 - 1, fn="plan_chunk_f32"):
     if not os.path.exists(_lib.LIB_PATH):
         pytest.skip("library not built")
-    f = getattr(ctypes.CDLL(_lib.LIB_PATH), "_ZN2qr14plan_chunk_f32ERKNS_9ChunkArgsE")
+    f = getattr(ctypes.CDLL(_lib.LIB_PATH), f"_ZN2qr{len(fn)}{fn}ERKNS_9ChunkArgsE")
     f.restype, f.argtypes = Plan, [ctypes.POINTER(Args)]
     a = Args()
     a.geom.planes, a.geom.kv_heads, a.geom.head_dim = 2, kv_heads, D
-    a.kv_dtype, a.heads, a.pos0, a.nq = dtype, heads, pos0, nq
+    a.kv_dtype, a.heads, a.pos0, a.nq, a.room = dtype, heads, pos0, nq, room
     p = f(ctypes.byref(a))
-    assert p.splits == 1 or p.workspace_bytes == nq * heads * p.splits * (4 * D + 8)
-    assert p.qblocks * p.queries_per_block >= nq and (64 // p.pg) // (heads // kv_heads) == p.queries_per_block
+    assert p.workspace_bytes == (nq * heads * p.splits * (4 * D + 8) if p.splits > 1 else 0)
+    assert p.qblocks * p.queries_per_block >= nq
+    rows = 64 // p.pg if p.pg else 64 * p.nt
+    assert p.queries_per_block == rows // (heads // kv_heads)
     return p
 
 
@@ -43,6 +46,17 @@ def test_chunk_f32_partials_are_bounded(dtype, D):
         for nq in [65, 128, 333, 512, 1000, 4095, 4096, 4097, 5000, 20000] + list(range(1500, 1600, 7)):
             for pos0 in (0, 1536, 100000):
                 assert plan(dtype, heads, kv_heads, D, pos0, nq).workspace_bytes < 80e6, (heads, kv_heads, nq, pos0)
+
+
+@pytest.mark.parametrize("fn,dtype,heads,kv_heads,D", [("plan_chunk_f32", 0, 32, 8, 128), ("plan_chunk_f32", 1, 16, 16, 256),
+                                                       ("plan_chunk", 1, 24, 8, 128), ("plan_chunk", 2, 28, 4, 64)])
+def test_chunk_plans_fit_the_room(fn, dtype, heads, kv_heads, D):
+    """Fewer splits in less room, none without: what a captured call gets."""
+    want = plan(dtype, heads, kv_heads, D, 3000, 200, fn=fn)
+    assert want.splits > 1
+    for room in (0, 256, want.workspace_bytes // 2, want.workspace_bytes - 1, want.workspace_bytes):
+        got = plan(dtype, heads, kv_heads, D, 3000, 200, room, fn)
+        assert got.workspace_bytes <= room and (got.splits == want.splits) == (room == want.workspace_bytes)
 
 
 def test_chunk_f32_plans_of_measured_shapes():

@@ -253,6 +253,42 @@ def test_chunk_f32_tiles_large_values(gpu, dtype, heads, kv_heads, D):
     assert np.all(np.abs(out / Vd[0, 0] - 1) <= 5e-6)  # the fp32 sums' bound of the tests above
 
 
+@pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,warm,nq", [
+    ("f32", 32, 8, 128, 700, 1300, 300),    # the larger call is unsplit, the smaller wants three splits
+    ("f16", 24, 8, 96, 1500, 1200, 70),
+    ("f16", 24, 8, 128, 700, 1400, 300),    # 16-bit tiles of a group of three
+])
+def test_chunk_captured_after_a_larger_call(gpu, dtype, heads, kv_heads, D, pos0, warm, nq):
+    """A captured chunk that wants more splits than any call before it had uses fewer, as the
+    decode entries did not need a larger workspace either; every replay equals the eager result
+    within the tolerance of the tiles."""
+    import torch
+
+    n = pos0 + warm
+    Kb, _, Vb, _ = make(n, n, kv_heads * D, dtype)
+    q = torch.from_numpy(np.random.default_rng(n).standard_normal((warm, heads * D), dtype=np.float32)).to(gpu)
+    out, eager = torch.empty_like(q), torch.empty_like(q[:nq])
+    scale = 1 / math.sqrt(D)
+    with qr.PagedKvCache(1, heads, kv_heads, D, n, kv_dtype=dtype) as kv:
+        kv.AppendRange(0, 0, Kb, Vb, src_dtype=dtype)
+        kv.AttentionChunkDev(0, pos0, q, out, scale)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            kv.AttentionChunkDev(0, pos0, q[:nq], out[:nq], scale)
+        results = []
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            results.append(out[:nq].cpu().numpy())
+        kv.AttentionChunkDev(0, pos0, q[:nq], eager, scale)
+        torch.cuda.synchronize()
+        del graph
+    for r in results:
+        assert errors(r, eager.cpu().numpy())[1] <= 2e-5
+
+
 @pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq,q_dtype", [
     ("f16", 28, 4, 128, 0, 130, "f16"),      # group 7: 18 queries fill 126 of a block's 128 rows
     ("bf16", 24, 8, 64, 300, 131, "f32"),    # group 3, hi + lo queries
