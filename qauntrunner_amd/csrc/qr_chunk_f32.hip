@@ -598,8 +598,15 @@ bool chunk_f32_eligible(int kv_dtype, int head_dim, int heads, int kv_heads, int
     // 197 MB 29.6 against 26.9 and 81.5 against 47.7; more than 64 queries took several decode
     // launches (128 queries from scratch: 21.4 against 16.0).  head_dim 96 is ahead from the
     // start (4 queries, 500 keys: 25.8 against 18.8).
+    // One head per kv head gives the entries a third of the work per byte: 64 queries after 400 (226
+    // MB) took 17.2 as entries and 20.7 here (head_dim 128), 32 after 1000 (266 MB) 17.8 and 19.8 (64),
+    // 16 after 2000 (263 MB) 21.7 and 20.2; at head_dim 256, where two launches are still ahead, 64
+    // after 300 (174 MB in 16 bits, 8 heads) 23.8 and 27.7, 32 after 500 (271 MB, 16 heads) 30.3 and
+    // 30.8, 65 after 100 (141 MB in fp32) 27.9 and 32.9, 64 after 400 (453 MB in fp32) 28.9 and 31.8.
     const double bytes = 2.0 * nq * (pos0 + 0.5 * nq) * kv_heads * head_dim * (f32 ? 4 : 2);
-    return nq > 64 || head_dim == 96 || bytes >= 96e6;
+    if (head_dim == 96) return true;
+    if (heads > kv_heads) return nq > 64 || bytes >= 96e6;
+    return nq > (head_dim == 256 ? 128 : 64) || bytes >= (head_dim == 256 && f32 ? 500e6 : 280e6);
 }
 
 ChunkPlan plan_chunk_f32(const ChunkArgs& a) {

@@ -23,10 +23,14 @@ class Plan(ctypes.Structure):  # ChunkPlan
                [("workspace_bytes", ctypes.c_size_t)]
 
 
-def plan(dtype, heads, kv_heads, D, pos0, nq, room=2**64 - 1, fn="plan_chunk_f32"):
+def library():
     if not os.path.exists(_lib.LIB_PATH):
         pytest.skip("library not built")
-    f = getattr(ctypes.CDLL(_lib.LIB_PATH), f"_ZN2qr{len(fn)}{fn}ERKNS_9ChunkArgsE")
+    return ctypes.CDLL(_lib.LIB_PATH)
+
+
+def plan(dtype, heads, kv_heads, D, pos0, nq, room=2**64 - 1, fn="plan_chunk_f32"):
+    f = getattr(library(), f"_ZN2qr{len(fn)}{fn}ERKNS_9ChunkArgsE")
     f.restype, f.argtypes = Plan, [ctypes.POINTER(Args)]
     a = Args()
     a.geom.planes, a.geom.kv_heads, a.geom.head_dim = 2, kv_heads, D
@@ -57,6 +61,27 @@ def test_chunk_plans_fit_the_room(fn, dtype, heads, kv_heads, D):
     for room in (0, 256, want.workspace_bytes // 2, want.workspace_bytes - 1, want.workspace_bytes):
         got = plan(dtype, heads, kv_heads, D, 3000, 200, room, fn)
         assert got.workspace_bytes <= room and (got.splits == want.splits) == (room == want.workspace_bytes)
+
+
+@pytest.mark.parametrize("tiles,dtype,heads,kv_heads,D,pos0,nq", [
+    (False, 0, 8, 8, 128, 400, 64),   # 17.2 us as decode entries, 20.7 on the tiles
+    (False, 0, 16, 16, 64, 1000, 32),  # 17.8, 19.8
+    (False, 2, 8, 8, 256, 300, 64),   # 23.8, 27.7
+    (False, 2, 16, 16, 256, 100, 64),  # 24.4, 31.7
+    (False, 0, 8, 8, 256, 100, 65),   # 27.9, 32.9
+    (False, 2, 8, 8, 256, 100, 100),  # 30.8, 35.5
+    (True, 0, 16, 16, 128, 0, 65),    # 17.3, 15.6
+    (True, 0, 32, 8, 128, 400, 64),   # four heads per kv head
+    (True, 2, 16, 16, 256, 1000, 64),  # 81.5, 55.6
+    (True, 2, 16, 16, 256, 0, 200),   # 67.3, 58.8
+    (True, 1, 16, 16, 96, 0, 8),
+    (False, 1, 16, 16, 96, 0, 7),     # fewer rows than half a tile
+])
+def test_chunk_f32_route(tiles, dtype, heads, kv_heads, D, pos0, nq):
+    """The faster side of the line between decode entries and tiles where both were timed."""
+    f = getattr(library(), "_ZN2qr18chunk_f32_eligibleEiiiiii")
+    f.restype = ctypes.c_bool
+    assert f(dtype, D, heads, kv_heads, pos0, nq) == tiles
 
 
 def test_chunk_f32_plans_of_measured_shapes():

@@ -169,6 +169,8 @@ def causal_f64(K, V, q, heads, kv_heads, D, pos0, scale):
     ("f16", 40, 1, 256, 3000, 75, "f32"),
     ("f32", 24, 8, 256, 1000, 300, "f32"),   # 64 rows of 21 queries, split
     ("f32", 32, 8, 128, 700, 300, "f32"),
+    ("f32", 16, 16, 256, 100, 140, "f16"),   # group 1, head_dim 256, past its line
+    ("bf16", 16, 16, 256, 1000, 64, "f32"),
 ])
 def test_chunk_f32_tiles(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dtype):
     """fp32 arithmetic over the exactly decoded cache: fp32 sums over up to 5,000 keys, 5e-6
@@ -234,7 +236,7 @@ def test_chunk_f32_tiles_error_of_decode_entries(gpu, dtype, heads, kv_heads, D,
     assert a <= 1.05 * b
 
 
-@pytest.mark.parametrize("dtype,heads,kv_heads,D", [("f32", 8, 2, 64), ("f32", 16, 16, 128), ("f32", 16, 16, 256),
+@pytest.mark.parametrize("dtype,heads,kv_heads,D", [("f32", 8, 2, 64), ("f32", 16, 16, 128), ("f32", 16, 8, 256),
                                                      ("bf16", 24, 8, 96)])
 def test_chunk_f32_tiles_large_values(gpu, dtype, heads, kv_heads, D):
     """V near the top of the range.  Positions 0 to 31 have score 0, position 40 one of 7.5 log2
