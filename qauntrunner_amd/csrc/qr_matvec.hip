@@ -1741,16 +1741,33 @@ bool fp_wave_fits(const MatVecArgs& a) {
            reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.cols % 8 == 0;
 }
 
+// Vectors per wave, up to four, spread evenly: the fewest rounds of resident waves, where a wave's
+// serial walk takes 1, 1.3, 1.4 and 1.5 of the unshared one for one to four vectors.  Sharing saves
+// reads of the weights, but each vector's x takes LDS (F16: seven one-wave workgroups per CU at
+// one vector, four at four), and one workgroup past what fits costs a whole walk: 4096 x 4096 F16
+// with eight vectors took 30.6, 28.2, 33.9 and 23.1 us at one to four, 5632 x 2048 with five
+// 15.7, 16.5, 18.9 and 18.7, 8192 x 3072 F32 with twelve 153, 83, 62 and 49.
+template <int FMT>
+int fp_vectors(int workgroups, int nq) {
+    const int lds[4] = {FwGeom<FMT, 8, 1>::SLOT, FwGeom<FMT, 8, 2>::SLOT, FwGeom<FMT, 8, 3>::SLOT, FwGeom<FMT, 8, 4>::SLOT};
+    constexpr int kWalk[4] = {10, 13, 14, 15};
+    int best = 1;
+    long long least = 0;
+    for (int n = 1; n <= 4 && n <= nq; ++n) {
+        const int passes = (nq + n - 1) / n, nv = (nq + passes - 1) / passes;
+        const long long fit = 256LL * (160 * 1024 / (kFwSlots * lds[nv - 1]));
+        const long long cost = (static_cast<long long>(workgroups) * passes + fit - 1) / fit * kWalk[nv - 1];
+        if (least == 0 || cost < least) {
+            least = cost;
+            best = nv;
+        }
+    }
+    return best;
+}
+
 template <int FMT>
 hipError_t launch_fp_group(const MatVecArgs& a, const FwGroup& g, hipStream_t stream) {
-    // Vectors per wave: as few as keep every wave resident at once (six one-wave workgroups per
-    // CU at two vectors), up to four, spread evenly.  Sharing saves reads of the weights but
-    // makes each wave's serial walk longer: 2048-column F16 layers whose waves all fit (4
-    // vectors) took 61.4 us unshared and 66.7 at four per wave; 5632 rows x 30 vectors of BF16
-    // 343 unshared and 232 shared.
-    const int fit = static_cast<int>(std::max(1LL, 1536LL / std::max(1, g.start[g.n])));
-    const int least = std::min(4, (a.nq + fit - 1) / fit);
-    const int passes = (a.nq + least - 1) / least, nv = (a.nq + passes - 1) / passes;
+    const int nv = fp_vectors<FMT>(g.start[g.n], a.nq), passes = (a.nq + nv - 1) / nv;
     const dim3 grid(static_cast<unsigned>(g.start[g.n]), static_cast<unsigned>(passes));
     if (nv == 1) hipLaunchKernelGGL((matvec_fp_wave<FMT, 8, 1>), grid, dim3(64), 0, stream, a, g);
     else if (nv == 2) hipLaunchKernelGGL((matvec_fp_wave<FMT, 8, 2>), grid, dim3(64), 0, stream, a, g);
@@ -1769,6 +1786,10 @@ hipError_t launch_fp(const MatVecArgs& a, hipStream_t stream) {
     g.rows[0] = a.rows;
     g.y[0] = a.y;
     return launch_fp_group<FMT>(a, g, stream);
+}
+
+int matvec_fp_vectors(int fmt, int workgroups, int nq) {
+    return fmt == QR_FMT_F32 ? fp_vectors<QR_FMT_F32>(workgroups, nq) : fp_vectors<QR_FMT_F16>(workgroups, nq);
 }
 
 hipError_t launch_matvec(const MatVecArgs& a, hipStream_t stream) {

@@ -26,6 +26,9 @@ hipError_t launch_matvec(const MatVecArgs& a, hipStream_t stream);
 // matrix;
 // every y equals launch_matvec's.
 constexpr int kMatVecGroupMax = 4;
+// Vectors that a wave of the float formats takes of nq, for a grid of `workgroups` row blocks of
+// eight rows.
+int matvec_fp_vectors(int fmt, int workgroups, int nq);
 hipError_t launch_matvec_group(const MatVecArgs* a, int n, hipStream_t stream);
 
 }  // namespace qr
