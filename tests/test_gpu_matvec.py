@@ -114,6 +114,78 @@ def test_matvec_several_vectors(gpu, fmt, rows, cols, nq):
     assert_exact(got, want, f"{fmt} {rows}x{cols} nq{nq}")
 
 
+def run_repeated(fmt, rows, cols, nq, seed):
+    """Matrices of many rows: 997 rows of weights over and over (a prime, so that a row summed or
+    stored in another's place shows), the oracle on those.  y and the wanted y of each matrix, one
+    grouped call."""
+    code = quant.FMT[fmt]
+    raw, _ = quant.random_rows(code, 997, cols, seed, 0.05)
+    raw = raw.reshape(997, -1)
+    x = normal(seed + 1, (nq, cols))
+    base, xd = dev(raw), dev(x)
+    at = [torch.arange(r, device="cuda") % 997 for r in rows]
+    ws = [base[i].reshape(-1) for i in at]
+    ys = [torch.full((nq, r), float("nan"), device="cuda") for r in rows]
+    if len(rows) == 1:
+        qr.matvec_dev(ws[0], code, rows[0], cols, xd, ys[0])
+    else:
+        qr.matvec_group_dev(ws, code, list(rows), cols, xd, ys)
+    torch.cuda.synchronize()
+    want = np.stack([oracle.matvec(code, raw, cols, x[b]) for b in range(nq)])
+    return [(y.cpu().numpy(), want[:, i.cpu().numpy()]) for y, i in zip(ys, at)]
+
+
+@pytest.mark.parametrize("fmt,rows,cols,nq", [
+    # tiles of a workgroup and how many of their terms LDS holds: 30 of 12, 20 of 13, 30 of 14, 27 of
+    # 14, 33 of 22, 318 of 256, and a group of 30, 32 and 32 of 12
+    ("Q8_0", (15003,), 1024, 32),
+    ("Q8_0", (2500,), 4096, 31),
+    ("Q4_0", (15003,), 1024, 30),
+    ("Q4_K", (15003,), 1024, 27),
+    ("Q8_0", (4103,), 14336, 5),
+    ("Q4_0", (1300003,), 64, 1),
+    ("Q8_0", (9001, 3000, 2999), 1024, 32),
+])
+def test_matvec_terms_summed_in_several_flushes(gpu, fmt, rows, cols, nq):
+    """Workgroups whose tiles' terms do not fit LDS at once: summed after each full set and once
+    more for the rest."""
+    for m, (got, want) in enumerate(run_repeated(fmt, rows, cols, nq, seed=rows[0] + nq)):
+        assert_exact(got, want, f"{fmt} {rows[m]}x{cols} nq{nq}")
+
+
+@pytest.mark.parametrize("fmt,rows,nq", [
+    # two vectors per wave (the last wave of a row block has one), three (one) and four (three; two)
+    ("F16", 1021, 15), ("F16", 2043, 13), ("F16", 4093, 7),
+    ("BF16", 1021, 15), ("BF16", 2043, 13), ("BF16", 4093, 7),
+    ("F32", 1021, 17), ("F32", 1021, 29), ("F32", 4093, 11),
+])
+@pytest.mark.parametrize("cols", [72, 1032])
+def test_matvec_fp_vectors_of_a_wave(gpu, fmt, rows, nq, cols):
+    """Float formats whose waves take several vectors: every vector as alone, in the oracle's bits."""
+    (got, want), = run_repeated(fmt, (rows,), cols, nq, seed=rows + nq + cols)
+    assert_exact(got, want, f"{fmt} {rows}x{cols} nq{nq}")
+
+
+@pytest.mark.parametrize("fmt,nq", [("F16", 7), ("BF16", 7), ("F32", 11)])
+def test_matvec_fp_vectors_of_a_wave_extremes(gpu, fmt, nq):
+    """Infinities, NaN and huge values in some vectors of a wave of four (F16: sums that are not
+    finite are taken again with the exact decode): each equals the same vector alone."""
+    code, rows, cols = quant.FMT[fmt], 4093, 264
+    raw = np.random.default_rng(8).integers(0, 256, rows * quant.random_rows(code, 1, cols, 1, 0.05)[0].size, dtype=np.uint8)
+    x = normal(9, (nq, cols))
+    x[1, ::3] = -0.0
+    x[2, 5], x[2, 77] = np.inf, np.nan
+    x[4, 100] = -np.inf
+    x[5] *= np.float32(1e30)
+    w, xd = dev(raw), dev(x)
+    y = torch.empty((nq, rows), device="cuda")
+    qr.matvec_dev(w, code, rows, cols, xd, y)
+    for v in range(nq):
+        one = torch.empty((1, rows), device="cuda")
+        qr.matvec_dev(w, code, rows, cols, xd[v:v + 1].contiguous(), one)
+        assert_exact_nan(y[v].cpu().numpy(), one[0].cpu().numpy(), f"{fmt} vector {v}")
+
+
 @pytest.mark.parametrize("fmt", ["Q8_0", "Q4_0", "Q4_K", "F16", "BF16", "F32"])
 def test_matvec_several_vectors_extremes(gpu, fmt):
     """Infinities, NaN, zeros of both signs and huge values in x, and weights of random bytes:
