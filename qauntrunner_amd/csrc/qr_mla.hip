@@ -921,7 +921,9 @@ __global__ void __launch_bounds__(kFWaves * 64, 1) mla_f32_kernel(const MlaMK p)
         if (i + 1 < nt) load_tile(i + 1);
         __builtin_amdgcn_sched_barrier(0);  // the next tile's loads leave before the softmax
 
-        // ---- softmax: this lane's positions are t0 + 4q4 + r (lazy rescale, as above)
+        // ---- softmax: this lane's positions are t0 + 4q4 + r.  The maximum does not lag here, so that
+        // weights stay at or below 1 as in the generic kernel: fp32 latents above 2^120 would
+        // overflow under weights of 256.
         const int t0 = t_wave + kFStep * i;
         float s[4];
         float tmax = -INFINITY;
@@ -931,7 +933,7 @@ __global__ void __launch_bounds__(kFWaves * 64, 1) mla_f32_kernel(const MlaMK p)
             tmax = fmaxf(tmax, s[r]);
         }
         tmax = max_xor32(max_xor16(tmax));
-        const bool grow = tmax > m + kRescaleSlack;
+        const bool grow = tmax > m;
         const bool rescale = grow && m != -INFINITY;
         if (__builtin_amdgcn_ballot_w64(rescale)) {
             const float corr = rescale ? fast_exp2(m - tmax) : 1.f;

@@ -103,6 +103,26 @@ def test_mla_fp32_tiles(gpu, heads, kv_lora, rope, n, pos):
         assert u[-1].item() == 7.0
 
 
+@pytest.mark.parametrize("kv_lora,rope", [(512, 64), (256, 32)])
+def test_mla_fp32_tiles_large_values(gpu, kv_lora, rope):
+    """Latents near the top of the range: positions 0 to 63 have score 0, position 67 -- the second
+    tile of one wave -- 7.5 log2 units above and the others none to speak of, so that weights
+    against the first tile's maximum overflow (2^7.5 x 5e36) where weights of at most 1 do not.
+    Latents past position 127, in other splits, are zero."""
+    heads, n, scale, v = 128, 4096, 1 / math.sqrt(192), np.float32(5e36)
+    lat = np.zeros((n, kv_lora + rope), np.float32)
+    lat[:128, :kv_lora] = v
+    lat[:, kv_lora] = -100 / scale
+    lat[:64, kv_lora] = 0
+    lat[67, kv_lora] = 7.5 * math.log(2) / scale
+    qrp = np.zeros((heads, rope), np.float32)
+    qrp[:, 0] = 1
+    with qr.MlaLatentCache(1, kv_lora + rope, n, dtype="f32", rope=rope) as m:
+        m.AppendRange(0, 0, lat)
+        u = m.AbsorbedAttention(0, n - 1, np.zeros((heads, kv_lora), np.float32), qrp, scale)
+    assert np.all(np.abs(u / v - 1) <= 2e-5)  # the tolerance of the tiles above
+
+
 @pytest.mark.parametrize("rope", [0, 16])
 def test_mla_absorbed_equals_expanded_through_gpu(gpu, rope):
     """Cli/Commands.cs:2065-2152: q-absorb -> GPU latent attention -> W_UV equals the
