@@ -629,15 +629,18 @@ bool chunk_mfma_eligible(int kv_dtype, int head_dim, int heads, int kv_heads) {
 // positions (28 heads over 4, bf16) took 137 us with the append, here 51, with errors against
 // 64 bits of 4.3e-6 and 2.2e-6.  Few queries over few keys keep the decode entries, which one or
 // two launches of 64 serve, merged in the kernel.  By the K/V bytes that the entries would read
-// themselves: 64 queries at 135 MB 15.9 us as entries against 20.1 here (head_dim 64) and 23.4
-// against 20.4 (head_dim 128), 16 queries at 197 MB 26.3 against 19.1; 128 queries from scratch
-// 17.7 against 19.4, 500 69 against 34.
+// themselves, as entries and here: 32 to 64 queries of head_dim 128 at 165 MB 16.3 us and 23.3 (64,
+// 40 heads over 8), at 280 MB 19 and 25 (64, 28 over 4) or 22 and 23, at 430 MB 24 and 29 or 33 and
+// 26 (48, 40 over 8), at 550 MB 31 and 26 or more apart; head_dim 64 at 220 MB 17.8 and 19.0, level
+// at 280; 8 and 16 queries at 165 MB 21.5 and 23.1 or 21.3 and 27.3, at 220 MB ahead or level; 65 to
+// 128 queries at 220 MB 24.0 and 24.8, at 280 MB ahead (129 from scratch 20.4 and 18.0).
 bool chunk_mfma_split_eligible(int kv_dtype, int head_dim, int heads, int kv_heads, int pos0, int nq) {
     if (kv_dtype == QR_DTYPE_F32 || (head_dim != 64 && head_dim != 128) || heads % kv_heads) return false;
     const int g = heads / kv_heads;
     if (g > 64 || (g & (g - 1)) == 0) return false;
     const double bytes = 4.0 * nq * (pos0 + 0.5 * nq) * kv_heads * head_dim;
-    return nq > 128 || (nq > 1 && bytes >= 160e6);
+    const double line = nq < 32 ? 220e6 : nq <= 64 && head_dim == 128 ? 430e6 : 280e6;
+    return nq > 128 || (nq > 1 && bytes >= line);
 }
 
 ChunkPlan plan_chunk(const ChunkArgs& a) {

@@ -294,7 +294,8 @@ def test_chunk_captured_after_a_larger_call(gpu, dtype, heads, kv_heads, D, pos0
 @pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq,q_dtype", [
     ("f16", 28, 4, 128, 0, 130, "f16"),      # group 7: 18 queries fill 126 of a block's 128 rows
     ("bf16", 24, 8, 64, 300, 131, "f32"),    # group 3, hi + lo queries
-    ("bf16", 24, 8, 128, 5000, 9, "bf16"),   # one N tile (position halves), keys split
+    ("bf16", 24, 8, 128, 5000, 9, "bf16"),   # few queries over few keys: decode entries
+    ("bf16", 24, 8, 128, 7000, 9, "bf16"),   # one N tile, past the line of few queries
     ("f16", 20, 4, 64, 1000, 140, "f32"),    # group 5
     ("f16", 63, 1, 128, 5, 133, "f16"),      # group 63: one query per block of 64 rows, two of 128
 ])
@@ -320,8 +321,8 @@ def test_chunk_mfma_uneven_groups(gpu, dtype, heads, kv_heads, D, pos0, nq, q_dt
     ("bf16", 28, 4, 64, 500, 129, 510),   # the first block, splits of two tiles
     ("f16", 28, 4, 128, 0, 1200, 600),    # unsplit: masked and unmasked tiles in one workgroup
     ("bf16", 24, 8, 128, 300, 131, 372),
-    ("f16", 24, 8, 128, 5000, 9, 5004),   # one N tile: two waves per row group, half a tile each
-    ("bf16", 28, 4, 64, 9000, 18, 9001),
+    ("f16", 24, 8, 128, 7000, 9, 7004),   # one N tile: two waves per row group, half a tile each
+    ("bf16", 28, 4, 64, 13000, 18, 13001),
 ])
 @pytest.mark.parametrize("value", [np.inf, np.nan])
 def test_chunk_mfma_uneven_groups_unseen_infinities(gpu, dtype, heads, kv_heads, D, pos0, nq, bad, value):
@@ -345,7 +346,7 @@ def test_chunk_mfma_uneven_groups_unseen_infinities(gpu, dtype, heads, kv_heads,
 @pytest.mark.parametrize("dtype,heads,kv_heads,D,pos0,nq,q_dtype", [
     ("f16", 28, 4, 128, 0, 140, "f16"),
     ("bf16", 24, 8, 64, 300, 131, "f32"),
-    ("f16", 24, 8, 128, 5000, 9, "f32"),
+    ("f16", 24, 8, 128, 7000, 9, "f32"),
     ("bf16", 32, 8, 128, 100, 70, "bf16"),
     ("f16", 64, 8, 64, 900, 6, "f32"),
 ])
