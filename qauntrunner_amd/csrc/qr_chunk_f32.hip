@@ -591,22 +591,34 @@ bool chunk_f32_eligible(int kv_dtype, int head_dim, int heads, int kv_heads, int
     if (nq < 2 || static_cast<long long>(nq) * (heads / kv_heads) < kChunkF32MinRows) return false;
     const bool f32 = kv_dtype == QR_DTYPE_F32;
     if (head_dim != 96 && head_dim != 256 && !(f32 && (head_dim == 64 || head_dim == 128))) return false;
-    // Few queries over few keys: one decode launch (up to 64 entries, merged in the kernel)
-    // costs less than this kernel and its merge.  K/V bytes that the entries would read
-    // themselves: at 66 MB 18.7 us as decode entries against 19.8 here (4 queries, 2000 keys,
-    // head_dim 128, append included) and 42.6 against 46.9 (16, 500, 16-bit head_dim 256), at
-    // 197 MB 29.6 against 26.9 and 81.5 against 47.7; more than 64 queries took several decode
-    // launches (128 queries from scratch: 21.4 against 16.0).  head_dim 96 is ahead from the
-    // start (4 queries, 500 keys: 25.8 against 18.8).
-    // One head per kv head gives the entries a third of the work per byte: 64 queries after 400 (226
-    // MB) took 17.2 as entries and 20.7 here (head_dim 128), 32 after 1000 (266 MB) 17.8 and 19.8 (64),
-    // 16 after 2000 (263 MB) 21.7 and 20.2; at head_dim 256, where two launches are still ahead, 64
-    // after 300 (174 MB in 16 bits, 8 heads) 23.8 and 27.7, 32 after 500 (271 MB, 16 heads) 30.3 and
-    // 30.8, 65 after 100 (141 MB in fp32) 27.9 and 32.9, 64 after 400 (453 MB in fp32) 28.9 and 31.8.
+    // More than 64 queries took several decode launches (128 from scratch, 32 heads over 8: 21.4 us
+    // against 16.0 here).  Few queries over few keys: one launch of up to 64 entries, merged in the
+    // kernel, costs less than this kernel and its merge.  The lines are by the K/V bytes that the
+    // entries would read themselves (us as entries and here, the append included):
+    //   32 to 64 queries, two heads per kv head: 200 MB 16.0 and 19.4 (64 after 349, head_dim 128), 300
+    //   MB 18.2 and 19.5 or ahead; three: 200 MB 21.8 and 25.1; four and more: 100 MB 16.4 and 19.2, 140
+    //   ahead; head_dim 256, two heads: 200 MB 23.5 and 35.0, 300 MB 28.7 and 31.7 in fp32, 140 MB 29.0
+    //   and 30.5 in 16 bits;
+    //   fewer: 66 MB 18.7 and 19.8 (4 after 2000), 197 MB 29.6 and 26.9; very few rows leave CUs idle
+    //   here (4 queries of 8 heads over 1 after 48826: 34.0 and 36.6, head_dim 64);
+    //   one head per kv head, where the entries do a third of the work per byte: 64 after 400 (226 MB)
+    //   17.2 and 20.7 (head_dim 128), 32 after 1000 (266 MB) 17.8 and 19.8 (64), 16 after 2000 (263 MB)
+    //   21.7 and 20.2; at head_dim 256, where two launches are still ahead, 64 after 300 (174 MB in 16
+    //   bits, 8 heads) 23.8 and 27.7, 32 after 500 (271 MB, 16 heads) 30.3 and 30.8, 65 after 100 (141
+    //   MB in fp32) 27.9 and 32.9, 64 after 400 (453 MB in fp32) 28.9 and 31.8.
+    // The entries of head_dim 96 are slower (4 queries after 500, 32 heads over 8: 25.8 and 18.8); with
+    // one head per kv head they are ahead over few keys (32 after 300 16.3 and 18.4, 8 after 500 16.9
+    // and 18.9, 8 after 2000 26.9 and 18.7).
+    const int g = heads / kv_heads;
+    if (head_dim == 96) return nq > 64 || g > 1 || pos0 + nq > 540;
+    if (nq > (g == 1 && head_dim == 256 ? 128 : 64)) return true;
+    if (head_dim < 256 && nq * heads < 64) return false;
+    const bool wide32 = head_dim == 256 && f32;
+    double line = 96e6;
+    if (g == 1) line = wide32 ? 500e6 : 280e6;
+    else if (nq >= 32) line = g == 2 ? (wide32 ? 350e6 : head_dim == 256 ? 200e6 : 300e6) : g == 3 ? 210e6 : 140e6;
     const double bytes = 2.0 * nq * (pos0 + 0.5 * nq) * kv_heads * head_dim * (f32 ? 4 : 2);
-    if (head_dim == 96) return true;
-    if (heads > kv_heads) return nq > 64 || bytes >= 96e6;
-    return nq > (head_dim == 256 ? 128 : 64) || bytes >= (head_dim == 256 && f32 ? 500e6 : 280e6);
+    return bytes >= line;
 }
 
 ChunkPlan plan_chunk_f32(const ChunkArgs& a) {

@@ -89,11 +89,18 @@ def test_chunk_plans_fit_the_room(fn, dtype, heads, kv_heads, D):
     (False, 2, 16, 16, 256, 100, 64),  # 24.4, 31.7
     (False, 0, 8, 8, 256, 100, 65),   # 27.9, 32.9
     (False, 2, 8, 8, 256, 100, 100),  # 30.8, 35.5
+    (False, 0, 16, 8, 128, 349, 64),  # 16.0, 19.4
+    (False, 0, 16, 8, 256, 158, 64),  # 23.5, 35.0
+    (False, 1, 16, 8, 256, 158, 64),  # 23.6, 33.3
+    (False, 0, 24, 8, 128, 349, 64),  # 21.8, 25.1
+    (False, 0, 32, 8, 128, 158, 64),  # 16.4, 19.2
+    (False, 0, 8, 1, 64, 48826, 4),   # 34.0, 36.6
+    (False, 2, 8, 8, 96, 300, 32),    # 16.0, 19.4
     (True, 0, 16, 16, 128, 0, 65),    # 17.3, 15.6
     (True, 0, 32, 8, 128, 400, 64),   # four heads per kv head
     (True, 2, 16, 16, 256, 1000, 64),  # 81.5, 55.6
     (True, 2, 16, 16, 256, 0, 200),   # 67.3, 58.8
-    (True, 1, 16, 16, 96, 0, 8),
+    (True, 1, 16, 16, 96, 2000, 8),   # 26.9, 18.7
     (False, 1, 16, 16, 96, 0, 7),     # fewer rows than half a tile
 ])
 def test_chunk_f32_route(tiles, dtype, heads, kv_heads, D, pos0, nq):

@@ -164,7 +164,7 @@ def causal_f64(K, V, q, heads, kv_heads, D, pos0, scale):
     ("f32", 40, 1, 128, 900, 70, "f32"),     # split
     ("f32", 64, 1, 128, 0, 100, "bf16"),
     ("f32", 64, 1, 256, 0, 66, "f32"),
-    ("f32", 33, 1, 256, 2000, 20, "f32"),
+    ("f32", 33, 1, 256, 2000, 70, "f32"),
     ("bf16", 64, 1, 96, 30, 40, "bf16"),
     ("f16", 40, 1, 256, 3000, 75, "f32"),
     ("f32", 24, 8, 256, 1000, 300, "f32"),   # 64 rows of 21 queries, split
