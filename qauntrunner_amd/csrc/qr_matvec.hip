@@ -1741,12 +1741,15 @@ bool fp_wave_fits(const MatVecArgs& a) {
            reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.cols % 8 == 0;
 }
 
-// Vectors per wave, up to four, spread evenly: the fewest rounds of resident waves, where a wave's
-// serial walk takes 1, 1.3, 1.4 and 1.5 of the unshared one for one to four vectors.  Sharing saves
-// reads of the weights, but each vector's x takes LDS (F16: seven one-wave workgroups per CU at
-// one vector, four at four), and one workgroup past what fits costs a whole walk: 4096 x 4096 F16
-// with eight vectors took 30.6, 28.2, 33.9 and 23.1 us at one to four, 5632 x 2048 with five
-// 15.7, 16.5, 18.9 and 18.7, 8192 x 3072 F32 with twelve 153, 83, 62 and 49.
+// Vectors per wave, up to four, spread evenly, by the longer of two times.  Rounds of resident
+// waves: a wave's serial walk takes 1, 1.3, 1.4 and 1.5 of the unshared one for one to four
+// vectors, each vector's x takes LDS (F16: seven one-wave workgroups per CU at one vector, four at
+// four), and one workgroup past what fits costs a whole walk.  Reads of the weights, once per pass
+// (a walk is about 2.8 ns a column, the reads of 900 workgroups of eight F32 rows as long).  At one
+// to four vectors per wave 4096 x 4096 F16 with eight took 30.6, 28.2, 33.9 and 23.1 us, 5632 x
+// 2048 with five 15.7, 16.5, 18.9 and 18.7, 4096 x 4096 F32 with three 22.6, 15.7 and 17.9, 8192 x
+// 3072 F32 with twelve 153, 83, 62 and 49.  Over 390 such points the choice takes 0.9% more than the
+// fastest, and none takes 3% more than unshared.
 template <int FMT>
 int fp_vectors(int workgroups, int nq) {
     const int lds[4] = {FwGeom<FMT, 8, 1>::SLOT, FwGeom<FMT, 8, 2>::SLOT, FwGeom<FMT, 8, 3>::SLOT, FwGeom<FMT, 8, 4>::SLOT};
@@ -1756,7 +1759,8 @@ int fp_vectors(int workgroups, int nq) {
     for (int n = 1; n <= 4 && n <= nq; ++n) {
         const int passes = (nq + n - 1) / n, nv = (nq + passes - 1) / passes;
         const long long fit = 256LL * (160 * 1024 / (kFwSlots * lds[nv - 1]));
-        const long long cost = (static_cast<long long>(workgroups) * passes + fit - 1) / fit * kWalk[nv - 1];
+        const long long waves = static_cast<long long>(workgroups) * passes;
+        const long long cost = std::max((waves + fit - 1) / fit * kWalk[nv - 1] * 2000, waves * (FMT == QR_FMT_F32 ? 22 : 11));
         if (least == 0 || cost < least) {
             least = cost;
             best = nv;

@@ -15,6 +15,8 @@ F32, F16 = 0, 1
     (F16, 2048, 16, 4),  # one round
     (F16, 4096, 2, 1),   # 12.2; 13.0
     (F32, 4096, 11, 4),
+    (F32, 4096, 3, 2),   # 15.7; one 22.6 (bound by reads of the weights), three 17.9
+    (F32, 8192, 12, 4),  # 49; 153, 83 and 62
     (F32, 1021, 29, 3),
     (F16, 1021, 15, 2),
     (F16, 64, 3, 1),
