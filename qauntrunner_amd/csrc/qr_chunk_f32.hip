@@ -9,9 +9,10 @@
 // Bound by the fp32 MFMA rate (v_mfma_f32_16x16x4_f32: 256 flop per clk and CU, 153 TFLOP/s in
 // a large product).  As one decode entry per query, the path before, every query read its own
 // K/V: 512 queries after 1536 positions (32 heads over 8 kv heads, head_dim 128, 15 GFLOP: 98 us
-// at that rate) took 8 launches of 61 us, 506 us per call with the append; this kernel takes 152
-// and its merge 7 (157 per call).  The matrix units are busy 81% of the cycles in which waves
-// are resident (1.0 LDS conflict cycle per MFMA); the rest is the softmax and the tile barriers.
+// at that rate) took 8 launches of 61 us, 506 us per call with the append; in two splits here 158
+// (traced, which slows each: kernel 162, merge 7.5, append 6.6).  The matrix units are busy 77% of
+// the cycles in which waves are resident (1.0 LDS conflict cycle per MFMA); the rest is the sums,
+// the softmax and the tile barriers.
 // Error against 64-bit results there: 2.9e-7 (decode entries 3.15e-7).
 //
 // A row is one (query, query head) pair.  Workgroup = 4 waves; the K/V tile of 32 positions is

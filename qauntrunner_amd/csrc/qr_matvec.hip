@@ -1454,7 +1454,7 @@ MvLayout mv_layout(const MatVecArgs& a) {
         const int rmax = std::max(1, std::min(kMvMaxRows, kMvThreads * kMvStageBatch * 16 / rbytes));
         // Q6_K has one item per block, a chain of 256 products, so few rows leave most threads of a
         // tile idle (4 rows of 16 blocks: 64 of 256): four times the rows, down to 256 tiles (an
-        // 8B layer of one vector 202 -> 172 us, of 2048 columns 123 -> 76)
+        // 8B layer of one vector 201 -> 170 us, of 2048 columns 125 -> 78)
         L.R = static_cast<int>(std::max(1LL, std::min<long long>(rmax, a.rows / (a.fmt == QR_FMT_Q6_K ? 256 : 1024))));
         L.stride = (rbytes + 15) / 16 * 16 + 16;
         L.copy_bytes = 16;

@@ -771,9 +771,9 @@ __global__ void __launch_bounds__(256) mla_combine_wide_kernel(const MlaMK p) {
 // Bound by the fp32 MFMA rate (v_mfma_f32_16x16x4_f32, 256 flop per clk and CU, fp32 products
 // and sums as the generic kernel's FMAs): 128 heads over 4096 positions are 1.14 GFLOP, 7.4 us
 // at the 153 TFLOP/s of a large fp32 product.  The generic kernel read every row once per
-// head, one row per thread: 1092 us per call at that shape, this one with its merge 29.0
-// (25.9 + 4.0; two tiles per wave there, so the first loads of q~ and rows are half of it).
-// Error against 64-bit arithmetic there: 4.6e-7 (generic 1.4e-6).
+// head, one row per thread: 1092 us per call at that shape, this one with its merge 29.6
+// (traced 29.3 + 4.3; two tiles per wave there, so the first loads of q~ and rows are half of it).
+// Error against 64-bit arithmetic there: 4.4e-7 (generic 1.4e-6).
 //
 // Workgroup = 16 heads over one split; its four waves take 16-position tiles 4i + w and work
 // alone: scores, online softmax and the latent sum of a tile stay in one wave, which the MFMA
