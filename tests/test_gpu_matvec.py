@@ -119,11 +119,12 @@ def run_repeated(fmt, rows, cols, nq, seed):
     stored in another's place shows), the oracle on those.  y and the wanted y of each matrix, one
     grouped call."""
     code = quant.FMT[fmt]
-    raw, _ = quant.random_rows(code, 997, cols, seed, 0.05)
-    raw = raw.reshape(997, -1)
+    n = min(997, max(rows))
+    raw, _ = quant.random_rows(code, n, cols, seed, 0.05)
+    raw = raw.reshape(n, -1)
     x = normal(seed + 1, (nq, cols))
     base, xd = dev(raw), dev(x)
-    at = [torch.arange(r, device="cuda") % 997 for r in rows]
+    at = [torch.arange(r, device="cuda") % n for r in rows]
     ws = [base[i].reshape(-1) for i in at]
     ys = [torch.full((nq, r), float("nan"), device="cuda") for r in rows]
     if len(rows) == 1:
@@ -137,7 +138,8 @@ def run_repeated(fmt, rows, cols, nq, seed):
 
 @pytest.mark.parametrize("fmt,rows,cols,nq", [
     # tiles of a workgroup and how many of their terms LDS holds: 30 of 12, 20 of 13, 30 of 14, 27 of
-    # 14, 33 of 22, 318 of 256, and a group of 30, 32 and 32 of 12
+    # 14, 33 of 22, 318 of 256, and a group of 30, 32 and 32 of 12; 33 passes of four vectors, more
+    # than an XCD has slots for
     ("Q8_0", (15003,), 1024, 32),
     ("Q8_0", (2500,), 4096, 31),
     ("Q4_0", (15003,), 1024, 30),
@@ -145,6 +147,7 @@ def run_repeated(fmt, rows, cols, nq, seed):
     ("Q8_0", (4103,), 14336, 5),
     ("Q4_0", (1300003,), 64, 1),
     ("Q8_0", (9001, 3000, 2999), 1024, 32),
+    ("Q8_0", (301,), 14336, 132),
 ])
 def test_matvec_terms_summed_in_several_flushes(gpu, fmt, rows, cols, nq):
     """Workgroups whose tiles' terms do not fit LDS at once: summed after each full set and once
